@@ -37,6 +37,8 @@ SOURCES = [
     ("assemble.hip", DEVICE + ["-ffp-contract=off"]),
     ("pcg.hip", DEVICE + ["-ffp-contract=fast"]),
     ("cg.hip", DEVICE + ["-ffp-contract=off"]),
+    ("resident.hip", DEVICE + ["-ffp-contract=off"]),
+    ("resident_plan.cpp", ["-ffp-contract=off"]),
     ("normals.hip", DEVICE + ["-ffp-contract=off"]),
     ("contact.hip", DEVICE + ["-ffp-contract=off"]),
     ("collide.hip", DEVICE + ["-ffp-contract=off"]),

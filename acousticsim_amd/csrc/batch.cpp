@@ -41,10 +41,9 @@ static int group_min(bool shared_launches)
     return shared_launches ? 512 : 2048;
 }
 
-template <typename T> T *Batch::dalloc(size_t n)
+void *Batch::dalloc_raw(size_t bytes)
 {
     void *p = nullptr;
-    const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
     check(hipMalloc(&p, bytes), "hipMalloc");
     allocations_.push_back(p);
     device_bytes_ += bytes;
@@ -52,7 +51,7 @@ template <typename T> T *Batch::dalloc(size_t n)
     // the fill runs on the null stream, which does not order work on this
     // batch's non-blocking stream: finish it before a kernel can write here
     check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
-    return static_cast<T *>(p);
+    return p;
 }
 
 namespace
@@ -211,6 +210,7 @@ Batch::~Batch()
         (void)hipHostFree(host_spmv_list_);
     if (host_upd_list_)
         (void)hipHostFree(host_upd_list_);
+    free_resident();
     if (contact_dev_)
         (void)hipFree(contact_dev_);
     if (detect_count_dev_)
@@ -650,6 +650,7 @@ void Batch::build_layout()
     user_force_.assign(models_.size(), std::vector<double>());
     sched_pairs_.reserve(models_.size());
     lane_order_.reserve(models_.size());
+    solved_.reserve(models_.size());
     pred_launches_.reserve(models_.size());
     drag_vertex_.assign(models_.size(), -1);
     ydrag_.assign(models_.size(), 0.0f);
@@ -681,6 +682,8 @@ void Batch::build_layout()
     upload(d_.ie_rows, ie_rows);
     upload(d_.ie_factor, ie_factor);
     upload(d_.params, params);
+    if (kind_ == SolverKind::CG32 || kind_ == SolverKind::CG64)
+        build_resident(col, slice_off, slice_w, params);
     // initial state: rest positions, at rest
     for (int i = 0; i < n; i++)
     {
@@ -1212,11 +1215,13 @@ int Batch::plan_lanes()
     const bool lanes_rule = env ? std::atoi(env) != 0 : true;
     const int n = size();
     lanes_[0].members.clear();
-    if (!lanes_rule || !lanes_allowed_ || n < 8 || d_.n_groups > 0 ||
+    const int left = (int)std::count(solved_.begin(), solved_.end(), 0);
+    if (!lanes_rule || !lanes_allowed_ || left < 8 || left < n || d_.n_groups > 0 ||
         (int)pred_launches_.size() != n)
     {
         for (int i = 0; i < n; i++)
-            lanes_[0].members.push_back(i);
+            if (!solved_[i])
+                lanes_[0].members.push_back(i);
         return 1;
     }
     std::vector<int> &order = lane_order_;
@@ -1325,9 +1330,38 @@ bool Batch::lane_update(Lane &L, long long cap)
     return any;
 }
 
-void Batch::solve_cg()
+void Batch::take_stats(int i, const CgState &s)
+{
+    StepStats &st = stats_[i];
+    st.pcg_iterations = s.total;
+    st.outer_iterations = s.updates;
+    st.matrix_fp64 = s.w64;
+    st.rel_residual = s.bb > 0 ? std::sqrt(s.rr_true / s.bb) : std::sqrt(s.rr_true);
+    // launches this cloth needed: two per iteration and per true residual
+    pred_launches_[i] = 2LL * (s.total + s.updates) + 2;
+}
+
+void Batch::solve_cg(const std::function<void()> &again)
 {
     launch_cg_reset(d_, stream_);
+    // the cloths that one launch solves; the launches below take the others
+    solved_.assign(size(), 0);
+    if (resident_.parts > 0 && lanes_allowed_ && !resident_.given_up && solve_resident(again))
+    {
+        read_states(lanes_[0]);
+        bool all = true;
+        if ((int)pred_launches_.size() != size())
+            pred_launches_.assign(size(), 0);
+        for (int i = 0; i < size(); i++)
+        {
+            solved_[i] = resident_.count[i] > 0;
+            if (solved_[i])
+                take_stats(i, host_cg_[2 * i]);
+            all &= solved_[i] != 0;
+        }
+        if (all)
+            return;
+    }
     long long cap = 16;
     for (auto &m : models_)
         cap = std::max<long long>(cap, 4LL * m.cfg.solver_max_iters + 64);
@@ -1338,7 +1372,7 @@ void Batch::solve_cg()
         chunk_schedule(L);
         L.active.assign(size(), 0);
         for (int i : L.members)
-            L.active[i] = 1;
+            L.active[i] = !solved_[i];
         L.next = 0;
         L.launched = 0;
         L.blind = 0;
@@ -1410,19 +1444,11 @@ void Batch::solve_cg()
             check(hipStreamWaitEvent(stream_, lanes_[k].ev, 0), "hipStreamWaitEvent");
         drain.armed = false;
     }
-    pred_launches_.assign(size(), 0);
+    pred_launches_.resize(size(), 0);
     for (int k = 0; k < nl; k++)
         for (int i : lanes_[k].members)
-        {
-            const CgState &s = lanes_[k].host_cg[2 * i];
-            StepStats &st = stats_[i];
-            st.pcg_iterations = s.total;
-            st.outer_iterations = s.updates;
-            st.matrix_fp64 = s.w64;
-            st.rel_residual = s.bb > 0 ? std::sqrt(s.rr_true / s.bb) : std::sqrt(s.rr_true);
-            // launches this cloth needed: two per iteration and per true residual
-            pred_launches_[i] = 2LL * (s.total + s.updates) + 2;
-        }
+            if (!solved_[i])
+                take_stats(i, lanes_[k].host_cg[2 * i]);
 }
 
 void Batch::begin_step()
@@ -2264,7 +2290,7 @@ void Batch::step_noalloc(int nsteps)
         const auto t0 = std::chrono::steady_clock::now();
         launch_elements(d_, stream_);
         launch_assemble_rows(d_, stream_);
-        solve_cg();
+        solve_cg([] {});
         launch_update_positions(d_, stream_);
         check(hipGetLastError(), "step launch");
         check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
@@ -2286,7 +2312,18 @@ void Batch::step_noalloc(int nsteps)
 
 void Batch::step(int nsteps)
 {
-    if (!tuned_)
+    if (!tuned_ && all_resident())
+    {
+        // no SpMV launch to tune: the variant whose rounding the one-launch
+        // solve follows is the one that the environment fixes, else 1 lane
+        // per row, gathered, cached
+        int lpr, stage, nt;
+        fixed_variant(lpr, stage, nt);
+        d_.spmv_lpr = lpr ? lpr : 1;
+        d_.spmv_stage = stage == 1;
+        d_.spmv_nt = nt == 1;
+    }
+    else if (!tuned_)
         autotune();
     for (int n = 0; n < nsteps; n++)
     {
@@ -2298,13 +2335,16 @@ void Batch::step(int nsteps)
             prepare_user_inputs();
             const bool ct = upload_contacts();
             launch_elements(d_, stream_);
-            launch_assemble_rows(d_, stream_);
-            if (ct) // W += collision Hessian (BaraffCloth.cpp:293)
-                launch_contact_hessian(d_, contact_blocks_, c_widx_, c_diag_, c_h9_, stream_);
+            auto rows = [&] {
+                launch_assemble_rows(d_, stream_);
+                if (ct) // W += collision Hessian (BaraffCloth.cpp:293)
+                    launch_contact_hessian(d_, contact_blocks_, c_widx_, c_diag_, c_h9_, stream_);
+            };
+            rows();
             if (kind_ == SolverKind::RefPCG64)
                 solve_ref();
             else
-                solve_cg();
+                solve_cg(rows);
             if (ct) // repulsion on dx (BaraffCloth.cpp:147)
                 launch_repulsion(d_, contact_groups_, c_wgl_, c_chl_, c_lvl_, c_wgr_, c_rows_,
                                  c_ids_, c_rec_, stream_);

@@ -1,6 +1,7 @@
 // Device-resident batch of independent cloths and the host driver of one
 // implicit substep (cBaraffCloth::UpdatePos, BaraffCloth.cpp:90-163).
 #pragma once
+#include <functional>
 #include <memory>
 #include <string>
 #include <vector>
@@ -8,6 +9,7 @@
 #include "collide.h"
 #include "device.h"
 #include "model.h"
+#include "resident.h"
 
 namespace bw
 {
@@ -202,6 +204,7 @@ private:
     hipEvent_t lanes_start_ = nullptr;
     bool lanes_allowed_ = true; // false inside bw_batch_step_noalloc
     std::vector<int> lane_order_;
+    std::vector<char> solved_; // per cloth: this solve's one launch has solved it
     int plan_lanes();
     void open_lane(Lane &L);
     void close_lane(Lane &L);
@@ -219,7 +222,29 @@ private:
     std::vector<std::pair<long long, int>> sched_pairs_;
     int upload_lists(Lane &L);
     void solve_ref();
-    void solve_cg();
+    // the solve of the assembled system; again: assembles it a second time
+    // (after a one-launch solve that was given up)
+    void solve_cg(const std::function<void()> &again);
+    void take_stats(int i, const CgState &s);
+    // One-launch solves (resident_plan.cpp).  build_resident: the cloths
+    // that fit them as parts, given the layout's columns; solve_resident:
+    // one launch over those cloths, false when it was given up and all
+    // states are again those of a solve's start
+    void build_resident(const std::vector<int> &col, const std::vector<int> &slice_off,
+                        const std::vector<int> &slice_w, const std::vector<InstParams> &params);
+    bool solve_resident(const std::function<void()> &again);
+    bool all_resident() const;
+    void free_resident();
+    struct ResidentPlan
+    {
+        std::vector<int> first, count; // parts of cloth i: first[i], count[i] (0: not resident)
+        int parts = 0, most = 0;       // parts in all, and of the largest cloth
+        int sets_max = 0, halo_max = 0;
+        ResidentBatch *table = nullptr; // device, one entry
+        char *ctl = nullptr, *host_ctl = nullptr; // ResidentCtl and tickets: device, pinned
+        int lpr = 0, capacity = 0;      // resident workgroups for that variant
+        bool given_up = false;          // a launch was: the batch solves by launches since
+    } resident_;
     // contacts: device lists for the next step (false if there are none)
     bool upload_contacts();
     // user inputs: upload the next step's user forces and drag pins before
@@ -260,7 +285,11 @@ private:
     std::vector<int4> slice_info_; // host copy of d_.slice_info (list entries carry it)
     unsigned long long graph_clock_ = 0;
     std::vector<void *> allocations_;
-    template <typename T> T *dalloc(size_t n);
+    void *dalloc_raw(size_t bytes); // zeroed, freed with the batch
+    template <typename T> T *dalloc(size_t n)
+    {
+        return static_cast<T *>(dalloc_raw((n ? n : 1) * sizeof(T)));
+    }
     std::vector<int> host_slice_off_;
     std::vector<Contacts> contacts_;
     int contact_total_ = 0;          // contacts over all cloths

@@ -61,6 +61,7 @@
 #include <climits>
 #include <cstdlib>
 
+#include "cg_math.h"
 #include "device.h"
 #include "reduce.h"
 
@@ -68,54 +69,6 @@ namespace bw
 {
 namespace
 {
-
-// field-wise state copies: whole-struct copies make the compiler keep a
-// per-thread copy of the state in LDS or scratch
-template <typename SP> __device__ inline CgState load_state(SP p)
-{
-    CgState s;
-    s.rho = p->rho;
-    s.rr_ref = p->rr_ref;
-    s.bb = p->bb;
-    s.rr_true = p->rr_true;
-    s.rr = p->rr;
-    s.start = p->start;
-    s.first = p->first;
-    s.iter = p->iter;
-    s.total = p->total;
-    s.since = p->since;
-    s.updates = p->updates;
-    s.done = p->done;
-    s.breakdown = p->breakdown;
-    s.pending = p->pending;
-    s.force_check = p->force_check;
-    s.final_check = p->final_check;
-    s.w64 = p->w64;
-    s.stalls = p->stalls;
-    return s;
-}
-
-template <typename SP> __device__ inline void store_state(SP p, const CgState &s)
-{
-    p->rho = s.rho;
-    p->rr_ref = s.rr_ref;
-    p->bb = s.bb;
-    p->rr_true = s.rr_true;
-    p->rr = s.rr;
-    p->start = s.start;
-    p->first = s.first;
-    p->iter = s.iter;
-    p->total = s.total;
-    p->since = s.since;
-    p->updates = s.updates;
-    p->done = s.done;
-    p->breakdown = s.breakdown;
-    p->pending = s.pending;
-    p->force_check = s.force_check;
-    p->final_check = s.final_check;
-    p->w64 = s.w64;
-    p->stalls = s.stalls;
-}
 
 // SpMV variants: L lanes per row (1, 2 or 4; a workgroup of L wavefronts
 // covers one 64-row slice, lane phase j takes ELL slots j, j+L, ...), slot
@@ -152,29 +105,6 @@ template <int L, typename T> __device__ inline T phase_sum(T v)
         v += __shfl_xor(v, off, 64);
     return v;
 }
-
-// the solver vectors of precision T
-template <typename T> struct Vecs;
-template <> struct Vecs<float>
-{
-    __device__ static const float *W(const DeviceBatch &d) { return d.W32; }
-    __device__ static const float *P(const DeviceBatch &d) { return d.P32; }
-    __device__ static float *r(const DeviceBatch &d) { return d.r32; }
-    __device__ static float *z(const DeviceBatch &d) { return d.z32; }
-    __device__ static float *q(const DeviceBatch &d) { return d.q32; }
-    __device__ static float *d0(const DeviceBatch &d) { return d.d32[0]; }
-    __device__ static float *d1(const DeviceBatch &d) { return d.d32[1]; }
-};
-template <> struct Vecs<double>
-{
-    __device__ static const double *W(const DeviceBatch &d) { return d.W64; }
-    __device__ static const double *P(const DeviceBatch &d) { return d.P64; }
-    __device__ static double *r(const DeviceBatch &d) { return d.r64; }
-    __device__ static double *z(const DeviceBatch &d) { return d.z64; }
-    __device__ static double *q(const DeviceBatch &d) { return d.q64; }
-    __device__ static double *d0(const DeviceBatch &d) { return d.d64[0]; }
-    __device__ static double *d1(const DeviceBatch &d) { return d.d64[1]; }
-};
 
 // Sums of components comp[] of the previous launch's partials of a cloth
 // (slot 0: written by k_cg_update, 1: by k_cg_spmv), in every wavefront.

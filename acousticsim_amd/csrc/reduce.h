@@ -20,40 +20,48 @@ enum Part
     P_RR64 = 4, // FP64 true residual r64.r64
 };
 
-// v of the lane that DPP control CTRL selects (every lane active); a
-// double moves as its two halves
+// v of the lane that DPP control CTRL selects (every lane active and every
+// selected lane inside its row, so the bound control only spares the
+// compiler a register set to zero); a double moves as its two halves
 template <int CTRL> __device__ inline double dpp_lane(double v)
 {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true);
     return __hiloint2double(hi, lo);
 }
 
-// v of lane ^ 32 (M = 32) or lane ^ 16 (M = 16) through gfx950's lane swap
-// of two registers (halves of the wavefront, or pairs of 16-lane rows).
-// Given the same register twice, one of the two results holds the partner
-// lane's value in every lane; which one is read off the same swap of the
-// lane index.
-template <int M> __device__ inline double swap_lane(double v)
+// a[l] + a[l ^ M] in the lanes l with (l & M) == 0 and b[l] + b[l ^ M] in the
+// others, for M = 32 or 16, through gfx950's lane swap of two registers (the
+// first one's upper half, or odd 16-lane rows, with the second one's lower
+// half, or even rows): afterwards the first register holds both values'
+// even halves and the second one their odd halves.  The order of the two
+// terms differs between lanes; their sum does not.
+template <int M> __device__ inline double swap_add(double a, double b)
 {
-    const int lane = threadIdx.x & 63;
-    const int lo = __double2loint(v), hi = __double2hiint(v);
+    const int al = __double2loint(a), ah = __double2hiint(a);
+    const int bl = __double2loint(b), bh = __double2hiint(b);
     if constexpr (M == 32)
     {
-        const auto li = __builtin_amdgcn_permlane32_swap(lane, lane, false, false);
-        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-        return (int)li[0] == (lane ^ 32) ? __hiloint2double(h[0], l[0])
-                                         : __hiloint2double(h[1], l[1]);
+        const auto l = __builtin_amdgcn_permlane32_swap(al, bl, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(ah, bh, false, false);
+        return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
     }
     else
     {
-        const auto li = __builtin_amdgcn_permlane16_swap(lane, lane, false, false);
-        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-        return (int)li[0] == (lane ^ 16) ? __hiloint2double(h[0], l[0])
-                                         : __hiloint2double(h[1], l[1]);
+        const auto l = __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+        return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
     }
+}
+
+// the last four steps of wave_sum: the sum over each 16-lane row
+__device__ inline double row_sum(double v)
+{
+    v += dpp_lane<0x128>(v);                 // row_ror:8
+    v += dpp_lane<0x1B>(dpp_lane<0x141>(v)); // row_half_mirror, then quad_perm [3,2,1,0]
+    v += dpp_lane<0x4E>(v);                  // quad_perm [2,3,0,1]
+    v += dpp_lane<0xB1>(v);                  // quad_perm [1,0,3,2]
+    return v;
 }
 
 // Sum over the 64 lanes of a wavefront (all active), the same value in every
@@ -65,13 +73,17 @@ template <int M> __device__ inline double swap_lane(double v)
 // permutations for 2 and 1.
 __device__ inline double wave_sum(double v)
 {
-    v += swap_lane<32>(v);
-    v += swap_lane<16>(v);
-    v += dpp_lane<0x128>(v);                 // row_ror:8
-    v += dpp_lane<0x1B>(dpp_lane<0x141>(v)); // row_half_mirror, then quad_perm [3,2,1,0]
-    v += dpp_lane<0x4E>(v);                  // quad_perm [2,3,0,1]
-    v += dpp_lane<0xB1>(v);                  // quad_perm [1,0,3,2]
-    return v;
+    v = swap_add<32>(v, v);
+    v = swap_add<16>(v, v);
+    return row_sum(v);
+}
+
+// wave_sum of two values at once, a's in the lower 32 lanes and b's in the
+// upper ones: the first swap halves the work of the other five steps
+__device__ inline double wave_sum2(double a, double b)
+{
+    const double v = swap_add<32>(a, b);
+    return row_sum(swap_add<16>(v, v));
 }
 
 // block-wide sums of N values (N <= 8), result in every thread

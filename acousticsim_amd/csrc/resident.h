@@ -1,0 +1,79 @@
+// One-launch tolerance solves (resident.hip): the device layout of a batch's
+// cloths as parts, one workgroup each, and the launcher.
+#pragma once
+#include "device.h"
+
+namespace bw
+{
+
+// Slices (64 rows, one wavefront each) of a part, by the solver's precision,
+// and matrix slots of a row that its registers keep.  8 in the mixed form:
+// with 4, a cloth has twice the parts, and the exchange costs more than the
+// shorter chains save (125 x 125 5.9 us an iteration against 5.4, 257 x 257
+// 12.2 against 9.3; only some 65 x 65 cloths gain).  4 in FP64, whose blocks
+// fill twice the registers.
+constexpr int RS_WAVES32 = 8, RS_WAVES64 = 4;
+constexpr int resident_slices(bool fp32) { return fp32 ? RS_WAVES32 : RS_WAVES64; }
+constexpr int RS_SLOTS = 13;
+// longest halo of a part (rows), by the solver's precision: with the sums of
+// the largest cloth (resident_plan.cpp) it fits the CU's 160 KiB of LDS
+constexpr int RS_HALO32 = 2688, RS_HALO64 = 2176;
+// Slices slice0 .. slice0 + n_slices - 1 of a cloth, solved by one workgroup
+// with the cloth's other parts. halo_off / halo_n: the rows of other parts
+// that its rows read (ResidentBatch::halo_row).
+struct ResidentPart
+{
+    int inst, slice0, n_slices;
+    int sets;       // slices of the whole cloth (partial sums to add)
+    int set0;       // the cloth's first slice
+    int halo_off, halo_n;
+    int parts;      // workgroups of the cloth
+};
+
+// A batch as the kernel sees it (a device table of these: a launch may run
+// cloths of several batches)
+struct ResidentBatch
+{
+    DeviceBatch d;
+    const ResidentPart *part;
+    const int *halo_row;
+    // per ELL entry (indexed like col): its column's position in the part's
+    // direction array, own rows first, then the halo
+    const uint16_t *pos;
+    // exchange words, {tag, 32 bits of a value}: z of every row (3 values),
+    // the solution of every row (3 doubles), and the partial sums of every
+    // slice: d.q (1 double), r.z and r.r (2), those of a true residual (3)
+    unsigned long long *z, *x, *s_dq, *s_rz, *s_res;
+    unsigned *epoch; // per cloth: the last tag used
+};
+
+// Launch control, at the head of the ticket buffer
+struct ResidentCtl
+{
+    int next;     // next ticket
+    int aborted;  // 1: a wait ran out; the launch's cloths are not solved
+    int pad[2];
+};
+
+struct ResidentLaunch
+{
+    const ResidentBatch *table; // device
+    ResidentCtl *ctl;           // device; the tickets (int2 {batch, part}) follow it
+    int tickets;
+    int lpr;                    // the SpMV variant whose rounding it follows (1, 2 or 4)
+    int sets_max, halo_max;     // over the launch's parts (halo_max even)
+    int give_up;                // tests: abort a cloth after this many iterations (0: never)
+    unsigned long long wait_ticks; // of the 100 MHz clock, per wait
+};
+
+// dynamic LDS bytes of a launch
+size_t resident_lds(bool fp32, int sets_max, int halo_max);
+// workgroups of the launch that are resident at once on the current device
+// (0 when the kernel cannot run with that LDS)
+int resident_capacity(bool fp32, int lpr, size_t lds);
+void launch_resident(const ResidentLaunch &a, bool fp32, int grid, hipStream_t s);
+// solver states of a solve that is started again (after an aborted launch):
+// the solve start, with the history that k_cg_reset had given it
+void launch_cg_restart(const DeviceBatch &d, hipStream_t s);
+
+} // namespace bw

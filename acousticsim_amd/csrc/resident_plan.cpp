@@ -1,0 +1,248 @@
+// The host side of the one-launch tolerance solve (resident.hip): which
+// cloths of a batch it takes, their parts, and the launch.
+#include <algorithm>
+#include <cstdlib>
+#include <cstring>
+#include <mutex>
+#include <stdexcept>
+
+#include "batch.h"
+
+namespace bw
+{
+
+namespace
+{
+void check(hipError_t e, const char *what)
+{
+    if (e != hipSuccess)
+        throw std::runtime_error(std::string("HIP error in ") + what + ": " + hipGetErrorString(e));
+}
+
+int env_int(const char *name, int otherwise)
+{
+    const char *e = std::getenv(name);
+    return e ? std::atoi(e) : otherwise;
+}
+
+// Limits of a cloth that is solved in one launch, such that any cloths
+// within them fit a launch's LDS together (resident_lds): slices, and rows
+// of other parts that a part reads.
+constexpr int SETS_CAP = 1088;
+int halo_cap(bool fp32) { return fp32 ? RS_HALO32 : RS_HALO64; }
+// Iterations that one launch may take (a launch is not interrupted)
+constexpr int ITER_CAP = 1000000;
+
+// One such launch at a time on a device: its workgroups wait for one
+// another, so two launches that each held part of the chip would both wait.
+std::mutex &device_turn()
+{
+    static std::mutex turn[64];
+    int dev = 0;
+    check(hipGetDevice(&dev), "hipGetDevice");
+    return turn[dev & 63];
+}
+} // namespace
+
+// Parts of each cloth that fits: its slices in order, split evenly over as
+// few workgroups as hold them.  BW_RESIDENT=0 turns one-launch solves off.
+void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &slice_off,
+                           const std::vector<int> &slice_w,
+                           const std::vector<InstParams> &params)
+{
+    const bool fp32 = kind_ == SolverKind::CG32;
+    const int hold = resident_slices(fp32);
+    ResidentPlan &rp = resident_;
+    rp = ResidentPlan();
+    rp.first.assign(size(), 0);
+    rp.count.assign(size(), 0);
+    // (words are addressed by 32-bit byte offsets)
+    if (d_.n_rows > (1 << 26) || opt_.shared_launches || env_int("BW_RESIDENT", 1) == 0)
+        return;
+    std::vector<ResidentPart> part;
+    std::vector<int> halo_row, rows;
+    std::vector<uint16_t> pos(col.size(), 0);
+    // per row: the last part that met it outside its own rows, and its
+    // place in that part's halo
+    std::vector<int> met(d_.n_rows, -1);
+    std::vector<uint16_t> place(d_.n_rows, 0);
+    int stamp = -1;
+    for (int i = 0; i < size(); i++)
+    {
+        const int n = nslices_[i], count = (n + hold - 1) / hold;
+        if (n > SETS_CAP || params[i].group_count > 0 || params[i].max_iter > ITER_CAP)
+            continue;
+        const size_t part0 = part.size(), halo0 = halo_row.size();
+        int longest = 0, s = slice_base_[i];
+        for (int k = 0; k < count; k++)
+        {
+            ResidentPart p = {};
+            p.inst = i;
+            p.slice0 = s;
+            p.n_slices = n / count + (k < n % count);
+            p.sets = n;
+            p.set0 = slice_base_[i];
+            p.halo_off = (int)halo_row.size();
+            p.parts = count;
+            s += p.n_slices;
+            const int r0 = p.slice0 * SLICE, r1 = s * SLICE;
+            const size_t e0 = slice_off[p.slice0],
+                         e1 = slice_off[s - 1] + (size_t)slice_w[s - 1] * SLICE;
+            rows.clear();
+            stamp++;
+            for (size_t e = e0; e < e1; e++)
+            {
+                const int c = col[e];
+                if ((c < r0 || c >= r1) && met[c] != stamp)
+                {
+                    met[c] = stamp;
+                    rows.push_back(c);
+                }
+            }
+            p.halo_n = (int)rows.size();
+            longest = std::max(longest, p.halo_n);
+            if (longest > halo_cap(fp32))
+                break;
+            std::sort(rows.begin(), rows.end());
+            for (size_t h = 0; h < rows.size(); h++)
+                place[rows[h]] = (uint16_t)(hold * SLICE + h);
+            for (size_t e = e0; e < e1; e++)
+                pos[e] = col[e] >= r0 && col[e] < r1 ? (uint16_t)(col[e] - r0) : place[col[e]];
+            halo_row.insert(halo_row.end(), rows.begin(), rows.end());
+            part.push_back(p);
+        }
+        if (longest > halo_cap(fp32))
+        {
+            part.resize(part0);
+            halo_row.resize(halo0);
+            continue;
+        }
+        rp.first[i] = (int)part0;
+        rp.count[i] = count;
+        rp.most = std::max(rp.most, count);
+        rp.sets_max = std::max(rp.sets_max, n);
+        rp.halo_max = std::max(rp.halo_max, (longest + 1) & ~1);
+    }
+    rp.parts = (int)part.size();
+    if (rp.parts == 0)
+        return;
+    auto put = [](auto *dst, const auto &v) {
+        if (!v.empty())
+            check(hipMemcpy(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice),
+                  "hipMemcpy H2D");
+    };
+    typedef unsigned long long u64;
+    auto *d_part = dalloc<ResidentPart>(part.size());
+    auto *d_halo = dalloc<int>(halo_row.size());
+    auto *d_pos = dalloc<uint16_t>(pos.size());
+    put(d_part, part);
+    put(d_halo, halo_row);
+    put(d_pos, pos);
+    ResidentBatch rb;
+    rb.d = d_;
+    rb.part = d_part;
+    rb.halo_row = d_halo;
+    rb.pos = d_pos;
+    rb.z = dalloc<u64>((size_t)d_.n_rows * 3 * (fp32 ? 1 : 2));
+    rb.x = dalloc<u64>((size_t)d_.n_rows * 6);
+    rb.s_dq = dalloc<u64>((size_t)d_.n_slices * 2);
+    rb.s_rz = dalloc<u64>((size_t)d_.n_slices * 4);
+    rb.s_res = dalloc<u64>((size_t)d_.n_slices * 6);
+    rb.epoch = dalloc<unsigned>(size());
+    rp.table = dalloc<ResidentBatch>(1);
+    check(hipMemcpy(rp.table, &rb, sizeof rb, hipMemcpyHostToDevice), "hipMemcpy H2D");
+    const size_t ctl = sizeof(ResidentCtl) + (size_t)rp.parts * sizeof(int2);
+    rp.ctl = dalloc<char>(ctl);
+    check(hipHostMalloc((void **)&rp.host_ctl, ctl), "hipHostMalloc");
+}
+
+void Batch::free_resident()
+{
+    if (resident_.host_ctl)
+        (void)hipHostFree(resident_.host_ctl);
+    resident_.host_ctl = nullptr;
+}
+
+bool Batch::all_resident() const
+{
+    if (resident_.parts == 0 || resident_.given_up)
+        return false;
+    for (int c : resident_.count)
+        if (c == 0)
+            return false;
+    return true;
+}
+
+// One launch over the resident cloths, after the reset of their states on
+// the batch's stream.  Cloths go in the order of the iterations that they
+// took in the last solve, the most first (in the first solve: of their
+// slices), since a launch lasts as long as its last cloth.  Returns false
+// when the launch is not possible here or was given up (a wait ran out
+// because other work kept the chip from holding a cloth's workgroups at
+// once): then `again` has assembled the system a second time, every state is
+// that of a solve's start, and the batch solves by launches from now on.
+bool Batch::solve_resident(const std::function<void()> &again)
+{
+    const bool fp32 = kind_ == SolverKind::CG32;
+    ResidentPlan &rp = resident_;
+    const size_t lds = resident_lds(fp32, rp.sets_max, rp.halo_max);
+    if (rp.lpr != d_.spmv_lpr)
+    {
+        rp.lpr = d_.spmv_lpr;
+        rp.capacity = resident_capacity(fp32, rp.lpr, lds);
+    }
+    if (rp.capacity < rp.most)
+    {
+        rp.given_up = true;
+        return false;
+    }
+    std::vector<int> &order = lane_order_;
+    order.clear();
+    for (int i = 0; i < size(); i++)
+        if (rp.count[i] > 0)
+            order.push_back(i);
+    const bool known = (int)pred_launches_.size() == size();
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+        return known ? pred_launches_[a] > pred_launches_[b] : nslices_[a] > nslices_[b];
+    });
+    ResidentCtl *ctl = reinterpret_cast<ResidentCtl *>(rp.host_ctl);
+    *ctl = ResidentCtl{};
+    int2 *ticket = reinterpret_cast<int2 *>(ctl + 1);
+    for (int i : order)
+        for (int k = 0; k < rp.count[i]; k++)
+            *ticket++ = make_int2(0, rp.first[i] + k);
+    ResidentLaunch a = {};
+    a.table = rp.table;
+    a.ctl = reinterpret_cast<ResidentCtl *>(rp.ctl);
+    a.tickets = rp.parts;
+    a.lpr = rp.lpr;
+    a.sets_max = rp.sets_max;
+    a.halo_max = rp.halo_max;
+    // waits end after 2 s (BW_RESIDENT_WAIT_MS); BW_RESIDENT_GIVE_UP makes
+    // the launch give up at that many iterations (tests)
+    a.give_up = env_int("BW_RESIDENT_GIVE_UP", 0);
+    a.wait_ticks = 100000ULL * (unsigned)std::max(0, env_int("BW_RESIDENT_WAIT_MS", 2000));
+    int aborted = 0;
+    {
+        std::lock_guard<std::mutex> turn(device_turn());
+        check(hipMemcpyAsync(rp.ctl, rp.host_ctl,
+                             sizeof(ResidentCtl) + (size_t)rp.parts * sizeof(int2),
+                             hipMemcpyHostToDevice, stream_),
+              "hipMemcpyAsync tickets");
+        launch_resident(a, fp32, std::min(rp.parts, rp.capacity), stream_);
+        check(hipGetLastError(), "resident launch");
+        check(hipMemcpyAsync(rp.host_ctl, rp.ctl, sizeof(ResidentCtl), hipMemcpyDeviceToHost,
+                             stream_),
+              "hipMemcpyAsync control");
+        check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+        aborted = ctl->aborted;
+    }
+    if (!aborted)
+        return true;
+    rp.given_up = true;
+    again();
+    launch_cg_restart(d_, stream_);
+    return false;
+}
+
+} // namespace bw

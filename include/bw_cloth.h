@@ -238,10 +238,12 @@ int bw_assemble_system(bw_cloth *c, double *W, double *rhs);
 const char *bw_last_error(void);
 
 /* ---- batched stepping (no reference counterpart: many independent cloths
-   of uneven size stepped together; from the second step on, a batch of 8
-   or more cloths solves the ones that needed the most launches in chains
-   of their own on separate streams, with results bit-identical to one
-   chain) -------------------------------------------------------------- */
+   of uneven size stepped together.  Tolerance solves of cloths of up to
+   about 69,000 vertices (65,000 in FP64) take one launch for all such cloths
+   of the batch, unless another process keeps the device from running it;
+   the others go by launches per iteration, where from the second step on 8
+   or more cloths solve the ones that needed the most launches in chains of
+   their own on separate streams.  Results are bit-identical either way) -- */
 
 /* n cloths from n JSON configs; x0s[i] may be NULL */
 int bw_batch_create(const char *const *json_configs, const double *const *x0s,
@@ -286,7 +288,7 @@ int bw_batch_detect_contacts(bw_batch *bt, int i, const bw_body *b, int cloth_fi
    memory; it allocates no device or host memory (the batch, created
    beforehand, holds everything else).  The solver states are carried in and
    out, so results are those of bw_batch_step with the same SpMV variant:
-   the autotuner's pick if bw_batch_step or bw_batch_autotune ran before,
+   bw_batch_step's or the autotuner's pick if either ran before,
    else the variant the BW_SPMV_* environment variables fix or the default;
    it never tunes.  Limits: tolerance-mode "fem" batches (BW_ERR_STATE
    otherwise, and while contacts or user perturbations are pending);
@@ -320,7 +322,9 @@ int bw_batch_time_launch_floor(bw_batch *b, int reps, double *avg_us);
    batch's own system and keep the fastest, or the first variant in the
    order below (fewer lanes, gathered, cached first) that times within 3%
    of it, so that near-equal variants do not swap between runs; the first
-   bw_batch_step does this by itself.  A variant is 1, 2 or 4 lanes per matrix row; the
+   bw_batch_step does this by itself when a cloth of the batch solves by
+   launches (else it takes 1 lane per row, gathered, cached: the lane count
+   sets the rounding that one-launch solves follow).  A variant is 1, 2 or 4 lanes per matrix row; the
    direction vector gathered from memory per slot, or staged in LDS once
    per distinct column of a 64-row slice; matrix loads with or without the
    nontemporal hint.  lanes gets the lanes per row chosen, staged and
