@@ -570,6 +570,7 @@ void Batch::build_layout()
         d_.q64 = dalloc<double>(nv3);
         d_.partial = dalloc<double>(PARTS * (size_t)d_.n_blocks_wg);
         d_.state = dalloc<InstState>(n);
+        d_.cg = dalloc<CgState>(2 * (size_t)n); // one-launch solves
     }
     else if (kind_ == SolverKind::GpuForm)
     {
@@ -682,7 +683,7 @@ void Batch::build_layout()
     upload(d_.ie_rows, ie_rows);
     upload(d_.ie_factor, ie_factor);
     upload(d_.params, params);
-    if (kind_ == SolverKind::CG32 || kind_ == SolverKind::CG64)
+    if (kind_ != SolverKind::GpuForm)
         build_resident(col, slice_off, slice_w, params);
     // initial state: rest positions, at rest
     for (int i = 0; i < n; i++)
@@ -1063,8 +1064,27 @@ void Batch::clear_warm_start(int i)
     check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
 }
 
-void Batch::solve_ref()
+void Batch::solve_ref(const std::function<void()> &again)
 {
+    if (all_resident())
+    {
+        launch_cg_reset(d_, stream_);
+        if (solve_resident(again))
+        {
+            check(hipMemcpyAsync(host_cg_, d_.cg, 2 * sizeof(CgState) * models_.size(),
+                                 hipMemcpyDeviceToHost, stream_),
+                  "hipMemcpyAsync state");
+            check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+            if ((int)pred_launches_.size() != size())
+                pred_launches_.assign(size(), 0);
+            for (int i = 0; i < size(); i++)
+            {
+                take_stats(i, host_cg_[2 * i]);
+                stats_[i].outer_iterations = 1;
+            }
+            return;
+        }
+    }
     launch_reset_states(d_, stream_);
     launch_pcg_init64(d_, stream_);
     int chunk = chunk_for(last_launches_ > 0 ? last_launches_ : 32);
@@ -2342,7 +2362,7 @@ void Batch::step(int nsteps)
             };
             rows();
             if (kind_ == SolverKind::RefPCG64)
-                solve_ref();
+                solve_ref(rows);
             else
                 solve_cg(rows);
             if (ct) // repulsion on dx (BaraffCloth.cpp:147)

@@ -221,9 +221,9 @@ private:
     void chunk_schedule(Lane &L);
     std::vector<std::pair<long long, int>> sched_pairs_;
     int upload_lists(Lane &L);
-    void solve_ref();
     // the solve of the assembled system; again: assembles it a second time
     // (after a one-launch solve that was given up)
+    void solve_ref(const std::function<void()> &again);
     void solve_cg(const std::function<void()> &again);
     void take_stats(int i, const CgState &s);
     // One-launch solves (resident_plan.cpp).  build_resident: the cloths
@@ -242,7 +242,7 @@ private:
         int sets_max = 0, halo_max = 0;
         ResidentBatch *table = nullptr; // device, one entry
         char *ctl = nullptr, *host_ctl = nullptr; // ResidentCtl and tickets: device, pinned
-        int lpr = 0, capacity = 0;      // resident workgroups for that variant
+        int lpr = -1, capacity = 0;     // resident workgroups for that variant
         bool given_up = false;          // a launch was: the batch solves by launches since
     } resident_;
     // contacts: device lists for the next step (false if there are none)

@@ -60,7 +60,9 @@ struct ResidentLaunch
     const ResidentBatch *table; // device
     ResidentCtl *ctl;           // device; the tickets (int2 {batch, part}) follow it
     int tickets;
-    int lpr;                    // the SpMV variant whose rounding it follows (1, 2 or 4)
+    // the rounding it follows: of the SpMV variant with 1, 2 or 4 lanes per
+    // row, or of the reference-semantics solver (0)
+    int lpr;
     int sets_max, halo_max;     // over the launch's parts (halo_max even)
     int give_up;                // tests: abort a cloth after this many iterations (0: never)
     unsigned long long wait_ticks; // of the 100 MHz clock, per wait

@@ -42,6 +42,13 @@
 // ResidentCtl::aborted, every workgroup leaves, and the host solves again by
 // launches.
 //
+// The reference's semantics (solver_mode "reference": FP64, exactly
+// max_iters - 1 iterations, BaraffCloth.cpp:529) are the same recurrences
+// with a tolerance of 0 and that cap, and the true residual after the last
+// iteration is the one that the counters report; REF gives it pcg.hip's
+// rounding, bit for bit.  65 x 65, 199 iterations, assembly included: 13.8
+// us an iteration by pcg.hip's launches, 6.4 here.
+//
 // Same rounding as cg.hip: a row's slots are added per lane phase of the
 // variant with L lanes per row, then the phases; a slice's partial sums in
 // that variant's order (slice_sum); a cloth's sums over its slices as
@@ -235,6 +242,25 @@ template <int L> __device__ inline double slice_sum(double v)
     return ((lane_value(v, 0) + lane_value(v, 16)) + lane_value(v, 32)) + lane_value(v, 48);
 }
 
+// The order of pcg.hip's reduce_cloth over the n sets of N sums in LDS (one a
+// solver workgroup there): a wavefront's worth of sets at a time, four of
+// those in turn.
+template <int N> __device__ inline void block_sets_sum(const double *sm, int n, double (&out)[N])
+{
+    const int lane = threadIdx.x & 63;
+    for (int j = 0; j < N; j++)
+        out[j] = 0.0;
+#pragma clang loop unroll(disable)
+    for (int g = 0; g < 4 && 64 * g < n; g++)
+        for (int j = 0; j < N; j++)
+        {
+            double t = 0.0;
+            for (int s = 64 * g + lane; s < n; s += 256)
+                t += sm[N * s + j];
+            out[j] += uniform(wave_sum(t));
+        }
+}
+
 // wave_sets_sum over the n sets of N sums in LDS, as scalars.  Four sets a
 // lane at a time; past the end zeros, which change no sum.
 template <int N> __device__ inline void sets_sum(const double *sm, int n, double (&out)[N])
@@ -279,6 +305,13 @@ template <int L, typename T> __device__ inline T phases(const T (&y)[L])
         return (y[0] + y[1]) + (y[2] + y[3]);
 }
 
+// block_row, or the order in which pcg.hip's compiler fuses its sum of three
+// products: m2 v2 + (m0 v0 + (m1 v1))
+template <bool REF, typename T> __device__ inline T block(T m0, T m1, T m2, T v0, T v1, T v2)
+{
+    return REF ? fma_t(m2, v2, fma_t(m0, v0, m1 * v1)) : block_row<T>(m0, m1, m2, v0, v1, v2);
+}
+
 __device__ inline ResidentPart uniform_part(const ResidentPart &v)
 {
     ResidentPart p;
@@ -299,10 +332,13 @@ __device__ inline ResidentPart uniform_part(const ResidentPart &v)
 // LDS or memory, what is uniform in scalar registers, and addresses are
 // formed where they are used (here()); with spills to scratch the product
 // alone took 5,500 cycles an iteration instead of 1,150.
-template <typename T, int WAVES, int L>
+// REF: the reference's semantics with pcg.hip's rounding (T = double, L = 1):
+// its order of a block's three products, and one set of sums per workgroup.
+template <typename T, int WAVES, int L, bool REF>
 __global__ void __launch_bounds__(WAVES * 64)
 k_resident(ResidentLaunch a)
 {
+    static_assert(!REF || (WAVES == BW_SB && L == 1), "a part is one of pcg.hip's workgroups");
     constexpr int NT = WAVES * 64; // threads, and rows of a part
     constexpr int NP = Pieces<T>::N;
     constexpr bool MIXED = sizeof(T) == sizeof(float);
@@ -355,6 +391,9 @@ k_resident(ResidentLaunch a)
         bool first = true;   // the next direction is P r
         bool w64 = uniform(sh_st.w64) != 0;
         bool check = true;   // a true residual is due (the warm start's)
+        // sets of sums: one a slice, or one a part
+        const int sets = REF ? pt.parts : pt.sets;
+        const int set_base = REF ? pt.set0 / BW_SB : pt.set0;
         const bool shared = pt.parts > 1;
         const bool have = wave < pt.n_slices; // this wavefront has a slice
         const int sl = pt.slice0 + (have ? wave : 0);
@@ -428,6 +467,22 @@ k_resident(ResidentLaunch a)
             const int l = here(lane), at = l / span;
             if (have && at < n && l % span == 0)
                 sm[n * (sl - pt.set0) + at] = v;
+            if constexpr (REF)
+            {
+                // pcg.hip's block_sum: the wavefronts in order
+                __syncthreads();
+                const int t = here(tid);
+                if (t >= 2 * n || (!shared && (t & 1)))
+                    return;
+                const double *from = sm + n * (pt.slice0 - pt.set0) + t / 2;
+                const double sum = ((from[0] + from[n]) + from[2 * n]) + from[3 * n];
+                if (!shared)
+                    sm[t / 2] = sum;
+                else
+                    word_store(word_at(words, 2 * n * (pt.slice0 / BW_SB) + t), tag,
+                               (unsigned)(t & 1 ? __double2hiint(sum) : __double2loint(sum)));
+                return;
+            }
             if (!shared)
                 return;
             __syncthreads();
@@ -443,8 +498,8 @@ k_resident(ResidentLaunch a)
             if (!shared)
                 return;
             unsigned *dst = reinterpret_cast<unsigned *>(sm);
-            G<u64> *w = words + (size_t)pt.set0 * n * 2;
-            const int count = pt.sets * n * 2;
+            G<u64> *w = words + (size_t)set_base * n * 2;
+            const int count = sets * n * 2;
             with_z = with_z && pt.halo_n > 0;
             const int e = here(tid);
             auto at = [&](int h) { return halo_word(words_z, e, h); };
@@ -457,6 +512,13 @@ k_resident(ResidentLaunch a)
                 in_time = pull_words<5, NT>(w, count, tag, dst, patience, hz, z_tag, at, with_z);
             if (!in_time)
                 sh_failed = 1;
+        };
+        auto total = [&](const double *sm, auto &out) {
+            constexpr int N = sizeof(out) / sizeof(out[0]);
+            if constexpr (REF)
+                block_sets_sum<N>(sm, sets, out);
+            else
+                sets_sum<N>(sm, sets, out);
         };
         // the slice's rows of W64 times the vectors v of the LDS array, in
         // the order of the variant with L lanes per row
@@ -473,9 +535,9 @@ k_resident(ResidentLaunch a)
                         const auto *x = v + 3 * (int)pos[(k0 + j) * SLICE];
                         const G<double> *w = W64 + 9 * (k0 + j) * SLICE;
                         for (int i = 0; i < 3; i++)
-                            y[i][j] += block_row<double>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
-                                                         w[(3 * i + 2) * SLICE], (double)x[0],
-                                                         (double)x[1], (double)x[2]);
+                            y[i][j] += block<REF>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
+                                                  w[(3 * i + 2) * SLICE], (double)x[0],
+                                                  (double)x[1], (double)x[2]);
                     }
             for (int i = 0; i < 3; i++)
                 sum[i] = phases<L>(y[i]);
@@ -551,7 +613,7 @@ k_resident(ResidentLaunch a)
                     break;
                 }
                 double t[3];
-                sets_sum<3>(sm_rz, pt.sets, t);
+                total(sm_rz, t);
                 rz = t[0];
                 rr = t[1];
                 // stop, or go on from the true residual (k_cg_spmv after a
@@ -588,6 +650,14 @@ k_resident(ResidentLaunch a)
                 }
             }
             const double beta = first ? 0.0 : uniform(rz / rho);
+            if (REF && !first && beta == 0.0)
+            {
+                // the reference stops here (BaraffCloth.cpp:585-590)
+                if (tid == 0)
+                    sh_st.final_check = 1;
+                check = true;
+                continue;
+            }
             rho = rz;
 
             // d = z + beta d_prev of the part's rows and of its halo
@@ -648,10 +718,9 @@ k_resident(ResidentLaunch a)
 #pragma unroll
                     for (int k = 0; k < N; k++)
                         for (int i = 0; i < 3; i++)
-                            y[i][(K0 + k) % L] += block_row<T>(m[K0 + k][3 * i],
-                                                               m[K0 + k][3 * i + 1],
-                                                               m[K0 + k][3 * i + 2], x[k][0],
-                                                               x[k][1], x[k][2]);
+                            y[i][(K0 + k) % L] +=
+                                block<REF>(m[K0 + k][3 * i], m[K0 + k][3 * i + 1],
+                                           m[K0 + k][3 * i + 2], x[k][0], x[k][1], x[k][2]);
                 };
                 slots(std::integral_constant<int, 0>(), std::integral_constant<int, 9>());
                 if (ws > 9)
@@ -666,8 +735,8 @@ k_resident(ResidentLaunch a)
                     const G<T> *w = glob(Vecs<T>::W(d)) + 9 * at + here(lane);
                     T t[3];
                     for (int i = 0; i < 3; i++)
-                        t[i] = block_row<T>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
-                                            w[(3 * i + 2) * SLICE], x[0], x[1], x[2]);
+                        t[i] = block<REF>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
+                                          w[(3 * i + 2) * SLICE], x[0], x[1], x[2]);
 #pragma unroll
                     for (int j = 0; j < L; j++)
                         if (k % L == j)
@@ -687,12 +756,12 @@ k_resident(ResidentLaunch a)
                 break;
             }
             double sq[1];
-            sets_sum<1>(sm_dq, pt.sets, sq);
+            total(sm_dq, sq);
             const double dq = sq[0];
-            if (!(dq > 0.0) || !isfinite(dq))
+            if (REF ? dq == 0.0 || !isfinite(dq) : !(dq > 0.0) || !isfinite(dq))
             {
-                // d.Wd == 0, or a loss of definiteness: stop after a final
-                // true residual
+                // d.Wd == 0 (BaraffCloth.cpp:547-551), or, to a tolerance, a
+                // loss of definiteness: stop after a final true residual
                 if (tid == 0)
                 {
                     sh_st.final_check = 1;
@@ -725,13 +794,13 @@ k_resident(ResidentLaunch a)
                 break;
             }
             double t[2];
-            sets_sum<2>(sm_rz, pt.sets, t);
+            total(sm_rz, t);
             rz = t[0];
             rr = t[1];
             steps++;
             first = false;
             // (NaN and infinity too)
-            check = (steps >= room) | !(rr > enough && rr < __builtin_inf());
+            check = (steps >= room) | (!REF && !(rr > enough && rr < __builtin_inf()));
         }
         if (failed)
         {
@@ -779,11 +848,14 @@ using ResidentKernel = void (*)(ResidentLaunch);
 
 template <int L> ResidentKernel kernel_for(bool fp32)
 {
-    return fp32 ? k_resident<float, RS_WAVES32, L> : k_resident<double, RS_WAVES64, L>;
+    return fp32 ? k_resident<float, RS_WAVES32, L, false> : k_resident<double, RS_WAVES64, L, false>;
 }
 
+// lpr 0: the reference's semantics
 ResidentKernel kernel_of(bool fp32, int lpr)
 {
+    if (lpr == 0)
+        return k_resident<double, RS_WAVES64, 1, true>;
     return lpr == 1 ? kernel_for<1>(fp32) : lpr == 2 ? kernel_for<2>(fp32) : kernel_for<4>(fp32);
 }
 

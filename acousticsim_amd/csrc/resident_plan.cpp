@@ -29,6 +29,8 @@ int env_int(const char *name, int otherwise)
 // within them fit a launch's LDS together (resident_lds): slices, and rows
 // of other parts that a part reads.
 constexpr int SETS_CAP = 1088;
+// Parts of a cloth: one per CU (resident_capacity is asked before a launch)
+constexpr int PARTS_CAP = 256;
 int halo_cap(bool fp32) { return fp32 ? RS_HALO32 : RS_HALO64; }
 // Iterations that one launch may take (a launch is not interrupted)
 constexpr int ITER_CAP = 1000000;
@@ -70,7 +72,7 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
     for (int i = 0; i < size(); i++)
     {
         const int n = nslices_[i], count = (n + hold - 1) / hold;
-        if (n > SETS_CAP || params[i].group_count > 0 || params[i].max_iter > ITER_CAP)
+        if (n > SETS_CAP || count > PARTS_CAP || params[i].group_count > 0 || params[i].max_iter > ITER_CAP)
             continue;
         const size_t part0 = part.size(), halo0 = halo_row.size();
         int longest = 0, s = slice_base_[i];
@@ -186,9 +188,10 @@ bool Batch::solve_resident(const std::function<void()> &again)
     const bool fp32 = kind_ == SolverKind::CG32;
     ResidentPlan &rp = resident_;
     const size_t lds = resident_lds(fp32, rp.sets_max, rp.halo_max);
-    if (rp.lpr != d_.spmv_lpr)
+    const int lpr = kind_ == SolverKind::RefPCG64 ? 0 : d_.spmv_lpr;
+    if (rp.lpr != lpr)
     {
-        rp.lpr = d_.spmv_lpr;
+        rp.lpr = lpr;
         rp.capacity = resident_capacity(fp32, rp.lpr, lds);
     }
     if (rp.capacity < rp.most)

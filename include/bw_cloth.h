@@ -238,9 +238,8 @@ int bw_assemble_system(bw_cloth *c, double *W, double *rhs);
 const char *bw_last_error(void);
 
 /* ---- batched stepping (no reference counterpart: many independent cloths
-   of uneven size stepped together.  Tolerance solves of cloths of up to
-   about 69,000 vertices (65,000 in FP64) take one launch for all such cloths
-   of the batch, unless another process keeps the device from running it;
+   of uneven size stepped together.  Solves of cloths of up to about 69,000
+   vertices (65,000 in FP64) take one launch for all such cloths of the batch, unless another process keeps the device from running it;
    the others go by launches per iteration, where from the second step on 8
    or more cloths solve the ones that needed the most launches in chains of
    their own on separate streams.  Results are bit-identical either way) -- */

@@ -102,3 +102,21 @@ def test_given_up_launch_solves_by_launches(monkeypatch):
     monkeypatch.setenv("BW_SPMV_NT", "0")
     _same(_run(monkeypatch, cloths, 2, "1", BW_RESIDENT_GIVE_UP="150"),
           _run(monkeypatch, cloths, 2, "0"))
+
+
+@pytest.mark.parametrize("rows,cols,max_iters", [(2, 2, 20), (9, 9, 1), (9, 9, 2), (16, 16, 90),
+                                                 (17, 16, 90), (33, 70, 150)])
+def test_reference_semantics_same_bits(monkeypatch, rows, cols, max_iters):
+    """the fixed iteration count in one launch against pcg.hip's launches"""
+    conf, x0 = _grid(rows, cols, "fp64")
+    del conf["precision"]
+    conf.update(solver_mode="reference", max_iters=max_iters)
+    a, b = (_run(monkeypatch, [(conf, x0), _reference_mesh(max_iters)], 2, r) for r in "10")
+    _same(a, b)
+
+
+def _reference_mesh(max_iters):
+    conf, x0 = _delaunay(700, "fp64")
+    del conf["precision"]
+    conf.update(solver_mode="reference", max_iters=max_iters)
+    return conf, x0
