@@ -89,7 +89,14 @@ std::vector<int> slice_row_order(const ClothModel &m)
         // 237 us (exact widths), 255 us (curve order only), 355 us (global
         // width sort).
         std::vector<int> order = hilbert_order(m.flat_xy);
-        int window = 65536; // BW_SORT_WINDOW overrides it for tuning runs
+        // Cloths that one launch solves (resident.hip) are cut into parts of
+        // 512 rows, and a window that tears a part's neighbourhood apart
+        // gives it a long halo: a 20,011-point mesh takes 8.8, 8.5 and 8.9 us
+        // an iteration with windows of 256, 512 and 1024 rows (7.0 with the
+        // blocks of its wide rows in LDS), and with 65536 its halos are too
+        // long for parts (11.2 us by launches).
+        const bool parts = (m.nv + SLICE - 1) / SLICE <= RS_SETS_CAP;
+        int window = parts ? RS_WAVES32 * SLICE : 65536; // BW_SORT_WINDOW: tuning runs
         if (const char *e = std::getenv("BW_SORT_WINDOW"))
             window = std::max(64, std::atoi(e));
         int bucket = 2; // widths compared in classes of this many slots

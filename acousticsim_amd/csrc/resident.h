@@ -15,6 +15,16 @@ namespace bw
 constexpr int RS_WAVES32 = 8, RS_WAVES64 = 4;
 constexpr int resident_slices(bool fp32) { return fp32 ? RS_WAVES32 : RS_WAVES64; }
 constexpr int RS_SLOTS = 13;
+// slices of the largest cloth that one launch solves
+constexpr int RS_SETS_CAP = 1088;
+// LDS of a part's workgroup at most, and of one more slot of its rows there
+// (nine values and a position)
+constexpr size_t RS_LDS_MAX = 160 * 1024 - 1024;
+constexpr size_t resident_slot_bytes(bool fp32)
+{
+    return (size_t)resident_slices(fp32) * SLICE *
+           (9 * (fp32 ? sizeof(float) : sizeof(double)) + sizeof(unsigned));
+}
 // longest halo of a part (rows), by the solver's precision: with the sums of
 // the largest cloth (resident_plan.cpp) it fits the CU's 160 KiB of LDS
 constexpr int RS_HALO32 = 2688, RS_HALO64 = 2176;
@@ -64,12 +74,13 @@ struct ResidentLaunch
     // row, or of the reference-semantics solver (0)
     int lpr;
     int sets_max, halo_max;     // over the launch's parts (halo_max even)
+    int extra;                  // slots past RS_SLOTS whose blocks are kept in LDS
     int give_up;                // tests: abort a cloth after this many iterations (0: never)
     unsigned long long wait_ticks; // of the 100 MHz clock, per wait
 };
 
 // dynamic LDS bytes of a launch
-size_t resident_lds(bool fp32, int sets_max, int halo_max);
+size_t resident_lds(bool fp32, int sets_max, int halo_max, int extra);
 // workgroups of the launch that are resident at once on the current device
 // (0 when the kernel cannot run with that LDS)
 int resident_capacity(bool fp32, int lpr, size_t lds);

@@ -25,13 +25,12 @@ int env_int(const char *name, int otherwise)
     return e ? std::atoi(e) : otherwise;
 }
 
-// Limits of a cloth that is solved in one launch, such that any cloths
-// within them fit a launch's LDS together (resident_lds): slices, and rows
-// of other parts that a part reads.
-constexpr int SETS_CAP = 1088;
+// Limit of a cloth that is solved in one launch, such that any cloths within
+// it and RS_SETS_CAP fit a launch's LDS together (resident_lds): rows of
+// other parts that a part reads.
+int halo_cap(bool fp32) { return fp32 ? RS_HALO32 : RS_HALO64; }
 // Parts of a cloth: one per CU (resident_capacity is asked before a launch)
 constexpr int PARTS_CAP = 256;
-int halo_cap(bool fp32) { return fp32 ? RS_HALO32 : RS_HALO64; }
 // Iterations that one launch may take (a launch is not interrupted)
 constexpr int ITER_CAP = 1000000;
 
@@ -46,8 +45,8 @@ std::mutex &device_turn()
 }
 } // namespace
 
-// Parts of each cloth that fits: its slices in order, split evenly over as
-// few workgroups as hold them.  BW_RESIDENT=0 turns one-launch solves off.
+// Parts of each cloth that fits: its slices in order, as many to a
+// workgroup as it holds.  BW_RESIDENT=0 turns one-launch solves off.
 void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &slice_off,
                            const std::vector<int> &slice_w,
                            const std::vector<InstParams> &params)
@@ -72,7 +71,7 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
     for (int i = 0; i < size(); i++)
     {
         const int n = nslices_[i], count = (n + hold - 1) / hold;
-        if (n > SETS_CAP || count > PARTS_CAP || params[i].group_count > 0 || params[i].max_iter > ITER_CAP)
+        if (n > RS_SETS_CAP || count > PARTS_CAP || params[i].group_count > 0 || params[i].max_iter > ITER_CAP)
             continue;
         const size_t part0 = part.size(), halo0 = halo_row.size();
         int longest = 0, s = slice_base_[i];
@@ -81,7 +80,7 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
             ResidentPart p = {};
             p.inst = i;
             p.slice0 = s;
-            p.n_slices = n / count + (k < n % count);
+            p.n_slices = std::min(hold, n - k * hold);
             p.sets = n;
             p.set0 = slice_base_[i];
             p.halo_off = (int)halo_row.size();
@@ -124,10 +123,14 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
         rp.most = std::max(rp.most, count);
         rp.sets_max = std::max(rp.sets_max, n);
         rp.halo_max = std::max(rp.halo_max, (longest + 1) & ~1);
+        for (int sl = slice_base_[i]; sl < slice_base_[i] + n; sl++)
+            rp.extra = std::max(rp.extra, slice_w[sl] - RS_SLOTS);
     }
     rp.parts = (int)part.size();
     if (rp.parts == 0)
         return;
+    const size_t used = resident_lds(fp32, rp.sets_max, rp.halo_max, 0);
+    rp.extra = std::min(rp.extra, (int)((RS_LDS_MAX - used) / resident_slot_bytes(fp32)));
     auto put = [](auto *dst, const auto &v) {
         if (!v.empty())
             check(hipMemcpy(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice),
@@ -187,7 +190,7 @@ bool Batch::solve_resident(const std::function<void()> &again)
 {
     const bool fp32 = kind_ == SolverKind::CG32;
     ResidentPlan &rp = resident_;
-    const size_t lds = resident_lds(fp32, rp.sets_max, rp.halo_max);
+    const size_t lds = resident_lds(fp32, rp.sets_max, rp.halo_max, rp.extra);
     const int lpr = kind_ == SolverKind::RefPCG64 ? 0 : d_.spmv_lpr;
     if (rp.lpr != lpr)
     {
@@ -221,6 +224,7 @@ bool Batch::solve_resident(const std::function<void()> &again)
     a.lpr = rp.lpr;
     a.sets_max = rp.sets_max;
     a.halo_max = rp.halo_max;
+    a.extra = rp.extra;
     // waits end after 2 s (BW_RESIDENT_WAIT_MS); BW_RESIDENT_GIVE_UP makes
     // the launch give up at that many iterations (tests)
     a.give_up = env_int("BW_RESIDENT_GIVE_UP", 0);
