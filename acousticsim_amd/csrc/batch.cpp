@@ -30,15 +30,16 @@ void check(hipError_t e, const char *what)
 // launches cost every iteration a little latency and save each large cloth
 // a redundant pass over its partials that grows with the square of its
 // slice count.  A batch's cloth may be solved alone and pay the latency in
-// full: 2048 (a 257 x 257 cloth, 1,032 slices, runs 23.7 steps/s without
-// group sums and 21.0 with).  The server's cloths always share their rounds'
-// launches: 512 (the serving mix runs 42.6 cloth-steps/s at 512 against
-// 32.0 at 2048).
+// full: 2048 (a 257 x 257 cloth, 1,032 slices, ran 23.7 steps/s without
+// group sums and 21.0 with).  The server's cloths share their rounds'
+// launches, where group sums pay off from 512 slices (a serving mix ran 42.6
+// cloth-steps/s at 512 against 32.0 at 2048); those that one launch solves
+// (resident.hip) have no use for them.
 static int group_min(bool shared_launches)
 {
     if (const char *e = std::getenv("BW_GROUP_MIN"))
         return std::max(0, std::atoi(e));
-    return shared_launches ? 512 : 2048;
+    return shared_launches ? RS_SETS_CAP : 2048;
 }
 
 void *Batch::dalloc_raw(size_t bytes)

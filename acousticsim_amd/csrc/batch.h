@@ -91,6 +91,17 @@ public:
     // the step counters and queues the position update.
     void begin_step();
     void end_step(const CgState *states, double step_us);
+    // between the two, for a one-cloth batch whose solve one launch may take
+    // (resident.h): its parts (0: none), its entry of the launch's table,
+    // what it asks of the launch's LDS, and, after a launch that was given
+    // up, the system and the state of the solve's start again (the batch
+    // has no parts from then on)
+    int resident_parts() const { return resident_.given_up ? 0 : resident_.parts; }
+    const ResidentBatch &resident_entry() const { return resident_.entry; }
+    int resident_sets() const { return resident_.sets_max; }
+    int resident_halo() const { return resident_.halo_max; }
+    int resident_extra_slots() const { return resident_.extra; }
+    void restart_step();
     size_t device_bytes() const { return device_bytes_; }
     // choose the SpMV variant by timing (done by the first step()); returns
     // the lanes per row picked; tune_us() has the times of variant v =
@@ -243,6 +254,7 @@ private:
         int extra = 0; // slots past the registers' that go to LDS
         ResidentBatch *table = nullptr; // device, one entry
         char *ctl = nullptr, *host_ctl = nullptr; // ResidentCtl and tickets: device, pinned
+        ResidentBatch entry = {};       // the table's
         int lpr = -1, capacity = 0;     // resident workgroups for that variant
         bool given_up = false;          // a launch was: the batch solves by launches since
     } resident_;

@@ -1,6 +1,8 @@
 // One-launch tolerance solves (resident.hip): the device layout of a batch's
 // cloths as parts, one workgroup each, and the launcher.
 #pragma once
+#include <mutex>
+
 #include "device.h"
 
 namespace bw
@@ -79,6 +81,15 @@ struct ResidentLaunch
     unsigned long long wait_ticks; // of the 100 MHz clock, per wait
 };
 
+// One such launch at a time on a device: its workgroups wait for one
+// another, so two launches that each held part of the chip would both wait.
+// Held from the launch until it has ended.
+std::mutex &resident_turn();
+// slots past RS_SLOTS that a launch can keep in LDS, of `wanted`
+int resident_extra(bool fp32, int sets_max, int halo_max, int wanted);
+// when a launch is given up: after a wait of 2 s (BW_RESIDENT_WAIT_MS), or at
+// BW_RESIDENT_GIVE_UP iterations of a cloth (tests)
+void resident_limits(ResidentLaunch &a);
 // dynamic LDS bytes of a launch
 size_t resident_lds(bool fp32, int sets_max, int halo_max, int extra);
 // workgroups of the launch that are resident at once on the current device

@@ -34,16 +34,27 @@ constexpr int PARTS_CAP = 256;
 // Iterations that one launch may take (a launch is not interrupted)
 constexpr int ITER_CAP = 1000000;
 
-// One such launch at a time on a device: its workgroups wait for one
-// another, so two launches that each held part of the chip would both wait.
-std::mutex &device_turn()
+} // namespace
+
+std::mutex &resident_turn()
 {
     static std::mutex turn[64];
     int dev = 0;
     check(hipGetDevice(&dev), "hipGetDevice");
     return turn[dev & 63];
 }
-} // namespace
+
+int resident_extra(bool fp32, int sets_max, int halo_max, int wanted)
+{
+    const size_t used = resident_lds(fp32, sets_max, halo_max, 0);
+    return std::min(wanted, (int)((RS_LDS_MAX - used) / resident_slot_bytes(fp32)));
+}
+
+void resident_limits(ResidentLaunch &a)
+{
+    a.wait_ticks = 100000ULL * (unsigned)std::max(0, env_int("BW_RESIDENT_WAIT_MS", 2000));
+    a.give_up = env_int("BW_RESIDENT_GIVE_UP", 0);
+}
 
 // Parts of each cloth that fits: its slices in order, as many to a
 // workgroup as it holds.  BW_RESIDENT=0 turns one-launch solves off.
@@ -58,7 +69,7 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
     rp.first.assign(size(), 0);
     rp.count.assign(size(), 0);
     // (words are addressed by 32-bit byte offsets)
-    if (d_.n_rows > (1 << 26) || opt_.shared_launches || env_int("BW_RESIDENT", 1) == 0)
+    if (d_.n_rows > (1 << 26) || env_int("BW_RESIDENT", 1) == 0)
         return;
     std::vector<ResidentPart> part;
     std::vector<int> halo_row, rows;
@@ -129,8 +140,6 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
     rp.parts = (int)part.size();
     if (rp.parts == 0)
         return;
-    const size_t used = resident_lds(fp32, rp.sets_max, rp.halo_max, 0);
-    rp.extra = std::min(rp.extra, (int)((RS_LDS_MAX - used) / resident_slot_bytes(fp32)));
     auto put = [](auto *dst, const auto &v) {
         if (!v.empty())
             check(hipMemcpy(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice),
@@ -154,6 +163,9 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
     rb.s_rz = dalloc<u64>((size_t)d_.n_slices * 4);
     rb.s_res = dalloc<u64>((size_t)d_.n_slices * 6);
     rb.epoch = dalloc<unsigned>(size());
+    rp.entry = rb;
+    if (opt_.shared_launches)
+        return; // the server has the table and the tickets
     rp.table = dalloc<ResidentBatch>(1);
     check(hipMemcpy(rp.table, &rb, sizeof rb, hipMemcpyHostToDevice), "hipMemcpy H2D");
     const size_t ctl = sizeof(ResidentCtl) + (size_t)rp.parts * sizeof(int2);
@@ -190,7 +202,8 @@ bool Batch::solve_resident(const std::function<void()> &again)
 {
     const bool fp32 = kind_ == SolverKind::CG32;
     ResidentPlan &rp = resident_;
-    const size_t lds = resident_lds(fp32, rp.sets_max, rp.halo_max, rp.extra);
+    const int extra = resident_extra(fp32, rp.sets_max, rp.halo_max, rp.extra);
+    const size_t lds = resident_lds(fp32, rp.sets_max, rp.halo_max, extra);
     const int lpr = kind_ == SolverKind::RefPCG64 ? 0 : d_.spmv_lpr;
     if (rp.lpr != lpr)
     {
@@ -224,14 +237,11 @@ bool Batch::solve_resident(const std::function<void()> &again)
     a.lpr = rp.lpr;
     a.sets_max = rp.sets_max;
     a.halo_max = rp.halo_max;
-    a.extra = rp.extra;
-    // waits end after 2 s (BW_RESIDENT_WAIT_MS); BW_RESIDENT_GIVE_UP makes
-    // the launch give up at that many iterations (tests)
-    a.give_up = env_int("BW_RESIDENT_GIVE_UP", 0);
-    a.wait_ticks = 100000ULL * (unsigned)std::max(0, env_int("BW_RESIDENT_WAIT_MS", 2000));
+    a.extra = extra;
+    resident_limits(a);
     int aborted = 0;
     {
-        std::lock_guard<std::mutex> turn(device_turn());
+        std::lock_guard<std::mutex> turn(resident_turn());
         check(hipMemcpyAsync(rp.ctl, rp.host_ctl,
                              sizeof(ResidentCtl) + (size_t)rp.parts * sizeof(int2),
                              hipMemcpyHostToDevice, stream_),
@@ -250,6 +260,14 @@ bool Batch::solve_resident(const std::function<void()> &again)
     again();
     launch_cg_restart(d_, stream_);
     return false;
+}
+
+void Batch::restart_step()
+{
+    resident_.given_up = true;
+    launch_assemble_rows(d_, stream_);
+    launch_cg_restart(d_, stream_);
+    check(hipGetLastError(), "step launch");
 }
 
 } // namespace bw

@@ -40,6 +40,9 @@ size_t estimate_bytes(const ClothModel &m)
     b += (size_t)m.nv * 4 * 4 + (size_t)m.nnzb() * 4 * 3;
     b += ((size_t)9 * m.nt + 16 * nie) * 4 + ((size_t)3 * m.nt + 4 * nie) * 4 * 2;
     b += (size_t)m.nt * (3 * 4 + 4 + 12 * 4 + 4 + 25 * 8) + nie * (4 * 4 + 8 + 25 * 8);
+    if (slices <= (size_t)RS_SETS_CAP) // one-launch solves: positions, exchange words, halos
+        b += entries * 2 + rows * (6 + 6) * 8 + slices * 12 * 8 +
+             slices * (sizeof(ResidentPart) + 4 * (size_t)RS_HALO32 / RS_WAVES64);
     return b + (1 << 20);
 }
 
@@ -67,6 +70,10 @@ Server::Server(const ServerOptions &opt) : opt_(opt), t0_(std::chrono::steady_cl
     check(hipHostMalloc((void **)&states_host_, ns * sizeof(CgState)), "hipHostMalloc");
     check(hipMalloc((void **)&table_dev_, opt_.max_resident * sizeof(DeviceBatch)), "hipMalloc");
     check(hipHostMalloc((void **)&table_host_, opt_.max_resident * sizeof(DeviceBatch)),
+          "hipHostMalloc");
+    check(hipMalloc((void **)&rs_table_dev_, opt_.max_resident * sizeof(ResidentBatch)),
+          "hipMalloc");
+    check(hipHostMalloc((void **)&rs_table_host_, opt_.max_resident * sizeof(ResidentBatch)),
           "hipHostMalloc");
     check(hipMemset(states_dev_, 0, ns * sizeof(CgState)), "hipMemset");
     check(hipStreamSynchronize(nullptr), "hipStreamSynchronize"); // before the server stream
@@ -98,6 +105,10 @@ Server::~Server()
     (void)hipStreamSynchronize(stream_);
     (void)hipFree(states_dev_);
     (void)hipFree(table_dev_);
+    (void)hipFree(rs_table_dev_);
+    (void)hipHostFree(rs_table_host_);
+    (void)hipFree(rs_ctl_dev_);
+    (void)hipHostFree(rs_ctl_host_);
     (void)hipFree(spmv_list_dev_);
     (void)hipFree(upd_list_dev_);
     (void)hipHostFree(states_host_);
@@ -282,13 +293,20 @@ void Server::builder_loop()
 void Server::upload_table(const std::vector<std::unique_ptr<Resident>> &res)
 {
     for (auto &r : res)
+    {
         table_host_[r->slot] = r->batch->device();
+        rs_table_host_[r->slot] = r->batch->resident_entry();
+    }
     // the whole table: slots are few and small
     int top = 0;
     for (auto &r : res)
         top = std::max(top, r->slot + 1);
     if (top > 0)
         check(hipMemcpyAsync(table_dev_, table_host_, top * sizeof(DeviceBatch),
+                             hipMemcpyHostToDevice, stream_),
+              "hipMemcpyAsync table");
+    if (top > 0)
+        check(hipMemcpyAsync(rs_table_dev_, rs_table_host_, top * sizeof(ResidentBatch),
                              hipMemcpyHostToDevice, stream_),
               "hipMemcpyAsync table");
     // one SpMV form per launch: staged when every resident request has its
@@ -406,25 +424,73 @@ void Server::retire(Resident &r, int error_code, const std::string &error)
     cv_budget_.notify_all();
 }
 
-int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
+// One launch takes the current step's solve of every request whose cloth
+// fits: the most iterations first (by the step before; in a first step the
+// largest cloth), since the launch lasts as long as its last cloth.
+bool Server::launch_one(std::vector<Resident *> &one, std::unique_lock<std::mutex> &turn)
 {
-    // start the next step of every resident request that is not solving
-    for (auto &r : res)
-        if (!r->solving)
-        {
-            r->batch->begin_step();
-            r->solving = true;
-            r->launched = 0;
-            r->t_step0 = now();
-            if (r->steps_done == 0)
-            {
-                std::lock_guard<std::mutex> lk(mu_);
-                info_[r->id].t_first = r->t_step0;
-            }
-        }
-    // lists of every solving request's slices and solver workgroups
+    ResidentLaunch a = {};
+    int most = 0, extra = 0;
+    for (Resident *r : one)
+    {
+        a.tickets += r->batch->resident_parts();
+        most = std::max(most, r->batch->resident_parts());
+        a.sets_max = std::max(a.sets_max, r->batch->resident_sets());
+        a.halo_max = std::max(a.halo_max, r->batch->resident_halo());
+        extra = std::max(extra, r->batch->resident_extra_slots());
+    }
+    a.lpr = opt_.spmv_lpr;
+    a.extra = resident_extra(opt_.fp32, a.sets_max, a.halo_max, extra);
+    const int capacity = resident_capacity(
+        opt_.fp32, a.lpr, resident_lds(opt_.fp32, a.sets_max, a.halo_max, a.extra));
+    if (capacity < most)
+        return false;
+    const size_t bytes = sizeof(ResidentCtl) + (size_t)a.tickets * sizeof(int2);
+    if (bytes > rs_ctl_cap_)
+    {
+        check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+        (void)hipFree(rs_ctl_dev_);
+        (void)hipHostFree(rs_ctl_host_);
+        rs_ctl_dev_ = rs_ctl_host_ = nullptr;
+        rs_ctl_cap_ = 0;
+        check(hipMalloc((void **)&rs_ctl_dev_, 2 * bytes), "hipMalloc");
+        check(hipHostMalloc((void **)&rs_ctl_host_, 2 * bytes), "hipHostMalloc");
+        rs_ctl_cap_ = 2 * bytes;
+    }
+    std::stable_sort(one.begin(), one.end(), [](const Resident *x, const Resident *y) {
+        if ((x->predicted > 0) != (y->predicted > 0))
+            return x->predicted == 0; // unknown: first
+        return x->predicted > 0 ? x->predicted > y->predicted
+                                : x->batch->device().n_slices > y->batch->device().n_slices;
+    });
+    ResidentCtl *ctl = reinterpret_cast<ResidentCtl *>(rs_ctl_host_);
+    *ctl = ResidentCtl{};
+    int2 *ticket = reinterpret_cast<int2 *>(ctl + 1);
+    for (Resident *r : one)
+        for (int k = 0; k < r->batch->resident_parts(); k++)
+            *ticket++ = make_int2(r->slot, k);
+    a.table = rs_table_dev_;
+    a.ctl = reinterpret_cast<ResidentCtl *>(rs_ctl_dev_);
+    resident_limits(a);
+    turn = std::unique_lock<std::mutex>(resident_turn());
+    check(hipMemcpyAsync(rs_ctl_dev_, rs_ctl_host_, bytes, hipMemcpyHostToDevice, stream_),
+          "hipMemcpyAsync tickets");
+    // (a sixteenth of the chip stays free for the builders' copies and fills)
+    launch_resident(a, opt_.fp32, std::min(a.tickets, std::max(most, capacity - capacity / 16)),
+                    stream_);
+    check(hipGetLastError(), "resident launch");
+    check(hipMemcpyAsync(rs_ctl_host_, rs_ctl_dev_, sizeof(ResidentCtl), hipMemcpyDeviceToHost,
+                         stream_),
+          "hipMemcpyAsync control");
+    return true;
+}
+
+// One chunk of launches over the requests `many`; its length.
+int Server::run_many(const std::vector<Resident *> &many)
+{
+    // lists of their slices and solver workgroups
     int n = 0, nb = 0, ng = 0;
-    for (auto &r : res)
+    for (Resident *r : many)
     {
         n += r->batch->device().n_slices;
         nb += r->batch->device().n_blocks_wg;
@@ -462,7 +528,7 @@ int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
         check(hipHostMalloc((void **)&upd_list_host_, list_cap_ * sizeof(int2)), "hipHostMalloc");
     }
     int k = 0, kb = 0;
-    for (auto &r : res)
+    for (Resident *r : many)
     {
         const DeviceBatch &d = r->batch->device();
         for (int s = 0; s < d.n_slices; s++)
@@ -475,7 +541,7 @@ int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
     for (; kb < ugrid; kb++)
         upd_list_host_[kb] = make_int2(-1, 0);
     int kg = 0;
-    for (auto &r : res)
+    for (Resident *r : many)
         for (int g = 0; g < r->batch->device().n_groups; g++)
             grp_list_host_[kg++] = make_int2(r->slot, g);
     for (; kg < ggrid; kg++)
@@ -492,12 +558,45 @@ int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
           "hipMemcpyAsync list");
     // run until the request expected to finish first should be done
     long long want = 1LL << 40;
-    for (auto &r : res)
+    for (Resident *r : many)
         want = std::min(want, r->predicted > r->launched ? r->predicted - r->launched : 64LL);
     const int length = (int)std::min<long long>(1024, std::max<long long>(32, (want + 31) / 32 * 32));
     run_chunk(length, grid, ggrid);
-    for (auto &r : res)
+    for (Resident *r : many)
         r->launched += length;
+    return length;
+}
+
+int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
+{
+    // start the next step of every resident request that is not solving
+    for (auto &r : res)
+        if (!r->solving)
+        {
+            r->batch->begin_step();
+            r->solving = true;
+            r->launched = 0;
+            r->t_step0 = now();
+            if (r->steps_done == 0)
+            {
+                std::lock_guard<std::mutex> lk(mu_);
+                info_[r->id].t_first = r->t_step0;
+            }
+        }
+    // the requests that one launch solves, and those that go by launches per
+    // iteration
+    std::vector<Resident *> one, many;
+    for (auto &r : res)
+        (r->batch->resident_parts() > 0 ? one : many).push_back(r.get());
+    std::unique_lock<std::mutex> turn;
+    if (!one.empty() && !launch_one(one, turn))
+    {
+        many.insert(many.end(), one.begin(), one.end());
+        one.clear();
+    }
+    int length = 0;
+    if (!many.empty())
+        length = run_many(many);
     // every slot's states in one copy
     int top = 0;
     for (auto &r : res)
@@ -506,10 +605,22 @@ int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
                          hipMemcpyDeviceToHost, stream_),
           "hipMemcpyAsync states");
     check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+    if (turn.owns_lock())
+        turn.unlock();
     {
         std::lock_guard<std::mutex> lk(mu_);
-        counters_.chunks++;
-        counters_.launches += length;
+        counters_.chunks += (one.empty() ? 0 : 1) + (many.empty() ? 0 : 1);
+        counters_.launches += (one.empty() ? 0 : 1) + length;
+    }
+    if (!one.empty() && reinterpret_cast<const ResidentCtl *>(rs_ctl_host_)->aborted)
+    {
+        // given up (resident.hip): these requests' steps start again and go
+        // by launches from now on
+        for (Resident *r : one)
+        {
+            r->batch->restart_step();
+            states_host_[2 * r->slot].done = 0;
+        }
     }
     // finish the steps whose solve is done
     std::vector<Resident *> finished, failed;

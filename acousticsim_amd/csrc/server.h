@@ -116,6 +116,7 @@ private:
     void builder_loop();
     void device_loop();
     int run_round(std::vector<std::unique_ptr<Resident>> &res);
+    int run_many(const std::vector<Resident *> &many);
     // final positions to the host (when error_code is BW_OK), device memory
     // and slot back, waiters woken
     void retire(Resident &r, int error_code, const std::string &error);
@@ -124,6 +125,15 @@ private:
     ServerOptions opt_;
     hipStream_t stream_ = nullptr;
     std::chrono::steady_clock::time_point t0_;
+
+    // One-launch solves of a round's requests that fit (resident.h): a table
+    // entry per slot, the launch's control and tickets
+    ResidentBatch *rs_table_dev_ = nullptr, *rs_table_host_ = nullptr;
+    char *rs_ctl_dev_ = nullptr, *rs_ctl_host_ = nullptr;
+    size_t rs_ctl_cap_ = 0;
+    // the launch for the requests `one`, its turn taken by `turn`; false
+    // when the device cannot hold one of them
+    bool launch_one(std::vector<Resident *> &one, std::unique_lock<std::mutex> &turn);
 
     // device tables
     CgState *states_dev_ = nullptr, *states_host_ = nullptr; // 2 per slot

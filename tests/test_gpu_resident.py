@@ -120,3 +120,23 @@ def _reference_mesh(max_iters):
     del conf["precision"]
     conf.update(solver_mode="reference", max_iters=max_iters)
     return conf, x0
+
+
+def test_served_same_bits(monkeypatch):
+    """requests solved together in one launch a round, also after a launch
+    that gives up mid-solve, against the batch's solver launches"""
+    cloths = [_grid(9, 9, "mixed", 0.2), _delaunay(1200, "mixed"), _grid(45, 45, "mixed", 5.0),
+              _grid(30, 31, "mixed")]
+    monkeypatch.setenv("BW_SPMV_LPR", "1")
+    monkeypatch.setenv("BW_SPMV_STAGE", "0")
+    monkeypatch.setenv("BW_SPMV_NT", "0")
+    ref = _run(monkeypatch, cloths, 2, "0")[0]
+    monkeypatch.setenv("BW_RESIDENT", "1")
+    for give_up in ("0", "150"):
+        monkeypatch.setenv("BW_RESIDENT_GIVE_UP", give_up)
+        s = capi.Server(budget_bytes=2e9, max_resident=8, precision="mixed")
+        ids = [s.submit(c, x, 2) for c, x in cloths]
+        for rid, x in zip(ids, ref):
+            assert s.wait(rid, 60.0) and s.info(rid)["status"] == 0
+            assert np.array_equal(s.get_pos(rid), x)
+        s.close()
