@@ -251,7 +251,7 @@ private:
         std::vector<int> first, count; // parts of cloth i: first[i], count[i] (0: not resident)
         int parts = 0, most = 0;       // parts in all, and of the largest cloth
         int sets_max = 0, halo_max = 0;
-        int extra = 0; // slots past the registers' that go to LDS
+        int extra = 0; // slots of slices past the registers' of a part
         ResidentBatch *table = nullptr; // device, one entry
         char *ctl = nullptr, *host_ctl = nullptr; // ResidentCtl and tickets: device, pinned
         ResidentBatch entry = {};       // the table's

@@ -19,13 +19,12 @@ constexpr int resident_slices(bool fp32) { return fp32 ? RS_WAVES32 : RS_WAVES64
 constexpr int RS_SLOTS = 13;
 // slices of the largest cloth that one launch solves
 constexpr int RS_SETS_CAP = 1088;
-// LDS of a part's workgroup at most, and of one more slot of its rows there
-// (nine values and a position)
+// LDS of a part's workgroup at most, and of one more slot of a slice there
+// (nine values and a position a row)
 constexpr size_t RS_LDS_MAX = 160 * 1024 - 1024;
 constexpr size_t resident_slot_bytes(bool fp32)
 {
-    return (size_t)resident_slices(fp32) * SLICE *
-           (9 * (fp32 ? sizeof(float) : sizeof(double)) + sizeof(unsigned));
+    return SLICE * (9 * (fp32 ? sizeof(float) : sizeof(double)) + sizeof(unsigned));
 }
 // longest halo of a part (rows), by the solver's precision: with the sums of
 // the largest cloth (resident_plan.cpp) it fits the CU's 160 KiB of LDS
@@ -76,7 +75,7 @@ struct ResidentLaunch
     // row, or of the reference-semantics solver (0)
     int lpr;
     int sets_max, halo_max;     // over the launch's parts (halo_max even)
-    int extra;                  // slots past RS_SLOTS whose blocks are kept in LDS
+    int extra;                  // slots of slices past RS_SLOTS that a part keeps in LDS
     int give_up;                // tests: abort a cloth after this many iterations (0: never)
     unsigned long long wait_ticks; // of the 100 MHz clock, per wait
 };
@@ -85,7 +84,7 @@ struct ResidentLaunch
 // another, so two launches that each held part of the chip would both wait.
 // Held from the launch until it has ended.
 std::mutex &resident_turn();
-// slots past RS_SLOTS that a launch can keep in LDS, of `wanted`
+// slots of slices past RS_SLOTS that a part can keep in LDS, of `wanted`
 int resident_extra(bool fp32, int sets_max, int halo_max, int wanted);
 // when a launch is given up: after a wait of 2 s (BW_RESIDENT_WAIT_MS), or at
 // BW_RESIDENT_GIVE_UP iterations of a cloth (tests)

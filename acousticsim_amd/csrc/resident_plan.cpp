@@ -134,8 +134,13 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
         rp.most = std::max(rp.most, count);
         rp.sets_max = std::max(rp.sets_max, n);
         rp.halo_max = std::max(rp.halo_max, (longest + 1) & ~1);
-        for (int sl = slice_base_[i]; sl < slice_base_[i] + n; sl++)
-            rp.extra = std::max(rp.extra, slice_w[sl] - RS_SLOTS);
+        for (size_t k = part0; k < part.size(); k++)
+        {
+            int extra = 0;
+            for (int sl = part[k].slice0; sl < part[k].slice0 + part[k].n_slices; sl++)
+                extra += std::max(0, slice_w[sl] - RS_SLOTS);
+            rp.extra = std::max(rp.extra, extra);
+        }
     }
     rp.parts = (int)part.size();
     if (rp.parts == 0)
