@@ -242,7 +242,12 @@ void Server::builder_loop()
             {
                 // allocations and copies on this thread would invalidate a
                 // graph the device thread is capturing
-                std::lock_guard<std::mutex> cap(capture_mu_);
+                struct Build
+                {
+                    CaptureGate &g;
+                    explicit Build(CaptureGate &gate) : g(gate) { g.enter_build(); }
+                    ~Build() { g.leave_build(); }
+                } build(gate_);
                 r->batch = std::make_unique<Batch>(std::move(ms), bo);
                 if (!job.x0.empty())
                 {
@@ -374,7 +379,12 @@ void Server::run_chunk(int length, int spmv_grid, int grp_grid)
             }
             hipGraph_t graph;
             {
-                std::lock_guard<std::mutex> cap(capture_mu_);
+                struct Capture
+                {
+                    CaptureGate &g;
+                    explicit Capture(CaptureGate &gate) : g(gate) { g.enter_capture(); }
+                    ~Capture() { g.leave_capture(); }
+                } cap(gate_);
                 check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal),
                       "BeginCapture");
                 launch_chain(piece, spmv_grid, grp_grid);

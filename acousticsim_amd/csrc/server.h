@@ -145,7 +145,43 @@ private:
     int grp_cap_ = 0;
 
     std::mutex mu_;
-    std::mutex capture_mu_; // graph capture vs. device allocations on the builder thread
+    // Device allocations and copies of the builder threads, which run side by
+    // side, against a graph capture on the device thread, which runs alone
+    // (they would invalidate it) and goes first when both wait.
+    class CaptureGate
+    {
+    public:
+        void enter_build()
+        {
+            std::unique_lock<std::mutex> lk(mu_);
+            cv_.wait(lk, [&] { return !capture_; });
+            builds_++;
+        }
+        void leave_build()
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            builds_--;
+            cv_.notify_all();
+        }
+        void enter_capture()
+        {
+            std::unique_lock<std::mutex> lk(mu_);
+            capture_ = true;
+            cv_.wait(lk, [&] { return builds_ == 0; });
+        }
+        void leave_capture()
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            capture_ = false;
+            cv_.notify_all();
+        }
+
+    private:
+        std::mutex mu_;
+        std::condition_variable cv_;
+        int builds_ = 0;
+        bool capture_ = false;
+    } gate_;
     std::condition_variable cv_jobs_, cv_ready_, cv_done_, cv_budget_;
     std::deque<Job> jobs_;
     std::deque<std::unique_ptr<Resident>> ready_;
