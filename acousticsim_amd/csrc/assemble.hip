@@ -7,7 +7,8 @@
 //   k_bend_elements : one thread per interior edge.  Dihedral angle beta and
 //     its gradient g (cDihedralMaterial::Update, DihedralBending.cpp:378-447);
 //     it stores l = factor * g, g and factor * beta.
-//   k_assemble_rows : one wavefront per ELL slice, one lane per block row.
+//   k_assemble_rows : one workgroup per ELL slice, one lane per block row, the
+//     row's slots dealt to the wavefronts.
 //     Each block W(v, c) = sk * (K_s + K_b) (+ sm * m_v I on the diagonal) is
 //     formed by summing its element contributions in ascending element order,
 //     exactly the order in which the reference's setFromTriplets sums
@@ -232,11 +233,27 @@ k_bend_elements(int n_ie, const int *__restrict__ ie_rows, const double *__restr
     out[24] = F * beta;
 }
 
-__global__ void __launch_bounds__(SLICE)
+// Wavefronts of a slice: a grid's rows have 13 slots, one each, and the last
+// wavefront has the force.  What bounds a row is its chain of dependent loads
+// (block -> list -> element record, per contribution), 25 us for the
+// diagonal's and 90 with all of a row's slots in one lane, and on a full chip
+// the chains that a CU holds at once.  So the slots run side by side, and a
+// block's lists and records are read ahead of the sums.  One wavefront a
+// slice without that, 8, 14: 5 x 5 vertices 91, 19, 20 us, 257 x 257 286, 206, 165, 600 x
+// 600 (0.5 GB written) 1588, 832, 779, 64 clothes of 256 to 16,384 vertices
+// 1851, 977, 912.
+constexpr int ROW_WAVES = 14;
+// Contributions to a block (to a force) whose records are read together: a
+// grid's diagonal block has 12 edges
+constexpr int TOGETHER = 4;
+
+__global__ void __launch_bounds__(ROW_WAVES *SLICE)
 k_assemble_rows(DeviceBatch d)
 {
+    __shared__ double diag[3][SLICE];
     const int s = blockIdx.x;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x % SLICE, wave = threadIdx.x / SLICE;
+    const bool last = wave == ROW_WAVES - 1; // the row's force and vectors too
     const int p = s * SLICE + lane;
     const int width = d.slice_w[s];
     const size_t base = (size_t)d.slice_off[s];
@@ -244,21 +261,59 @@ k_assemble_rows(DeviceBatch d)
     const InstParams &P = d.params[d.slice_inst[s]];
     double *W64 = d.W64 + 9 * base + lane;
     float *W32 = d.W32 + 9 * base + lane;
-    if (vg < 0)
+    const bool row = vg >= 0; // else padding
+    const bool pin_p = row && d.row_pinned[p] != 0;
+    const double mass = row ? d.row_mass[p] : 0.0;
+    const int b0 = row ? d.blk_ptr[vg] : 0, nb = row ? d.blk_ptr[vg + 1] - b0 : 0;
+    if (last)
+        for (int a = 0; a < 3; a++)
+            diag[a][lane] = 1.0;
+    __syncthreads();
+    // force: stretch sum over incident triangles, then bending over incident
+    // interior edges (CalcTotalForce BaraffMaterial.cpp:267-282,
+    // AssignForceAndMatrix DihedralBending.cpp:449-489)
+    double fs[3] = {0.0, 0.0, 0.0}, fb[3] = {0.0, 0.0, 0.0};
+    if (last && row)
     {
-        for (int k = 0; k < width; k++)
-            for (int q = 0; q < 9; q++)
+        const int t0 = d.vt_ptr[vg], t1 = d.vt_ptr[vg + 1];
+        const int e0 = d.ve_ptr[vg], e1 = d.ve_ptr[vg + 1];
+        for (int it = t0; it < t1; it += TOGETHER)
+        {
+            double f[TOGETHER][3];
+#pragma unroll
+            for (int u = 0; u < TOGETHER; u++)
             {
-                W64[(9 * k + q) * SLICE] = 0.0;
-                W32[(9 * k + q) * SLICE] = 0.0f;
+                const int code = d.vt_list[min(it + u, t1 - 1)];
+                const double *ing = d.tri_ing + (size_t)ING * (code >> 2) + 16 + 3 * (code & 3);
+                for (int a = 0; a < 3; a++)
+                    f[u][a] = ing[a];
             }
-        return;
+#pragma unroll
+            for (int u = 0; u < TOGETHER; u++)
+                if (it + u < t1)
+                    for (int a = 0; a < 3; a++)
+                        fs[a] = fs[a] + f[u][a];
+        }
+        for (int it = e0; it < e1; it += TOGETHER)
+        {
+            double beta[TOGETHER], g[TOGETHER][3];
+#pragma unroll
+            for (int u = 0; u < TOGETHER; u++)
+            {
+                const int code = d.ve_list[min(it + u, e1 - 1)];
+                const double *ing = d.ie_ing + (size_t)ING * (code >> 2);
+                beta[u] = ing[24];
+                for (int a = 0; a < 3; a++)
+                    g[u][a] = ing[12 + 3 * (code & 3) + a];
+            }
+#pragma unroll
+            for (int u = 0; u < TOGETHER; u++)
+                if (it + u < e1)
+                    for (int a = 0; a < 3; a++)
+                        fb[a] = fb[a] + (beta[u] * g[u][a]) / 2;
+        }
     }
-    const bool pin_p = d.row_pinned[p] != 0;
-    const double mass = d.row_mass[p];
-    const int b0 = d.blk_ptr[vg], nb = d.blk_ptr[vg + 1] - b0;
-    double diag[3] = {1.0, 1.0, 1.0};
-    for (int k = 0; k < width; k++)
+    for (int k = wave; k < width; k += ROW_WAVES)
     {
         double w[9];
         if (k < nb)
@@ -271,22 +326,38 @@ k_assemble_rows(DeviceBatch d)
                 ks[q] = 0.0;
                 kb[q] = 0.0;
             }
+            const int s0 = d.s_ptr[blk], s1 = d.s_ptr[blk + 1];
+            const int e0 = d.b_ptr[blk], e1 = d.b_ptr[blk + 1];
+            int next = s0 < s1 ? d.s_list[s0] : 0, edge[TOGETHER];
+            for (int u = 0; u < TOGETHER; u++)
+                edge[u] = e0 < e1 ? d.b_list[min(e0 + u, e1 - 1)] : 0;
             // stretch: (0 + H_warpweft) + H_bias per triangle, triangles ascending
-            for (int it = d.s_ptr[blk]; it < d.s_ptr[blk + 1]; it++)
+            for (int it = s0; it < s1; it++)
             {
-                const int code = d.s_list[it];
+                const int code = next;
+                next = d.s_list[min(it + 1, s1 - 1)];
                 const int t = code >> 4, i = (code >> 2) & 3, j = code & 3;
                 const double *ing = d.tri_ing + (size_t)ING * t;
                 const float *cf = d.tri_coef + 12 * (size_t)t;
                 const double A = (double)d.tri_area[t];
-                const InstParams &Pt = d.params[d.tri_inst[t]];
-                double h[9];
+                double rec[16], h[9];
+                float ci[4], cj[4];
+#pragma unroll
+                for (int q = 0; q < 16; q++)
+                    rec[q] = ing[q];
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                {
+                    ci[q] = cf[3 * q + i];
+                    cj[q] = cf[3 * q + j];
+                }
+#pragma unroll
                 for (int set = 0; set < 2; set++)
                 {
-                    const double Ku = set == 0 ? Pt.k0 : Pt.k2, Kv = set == 0 ? Pt.k1 : Pt.k2;
-                    const double su2 = (Ku * (double)cf[6 * set + i]) * (double)cf[6 * set + j];
-                    const double sv2 = (Kv * (double)cf[6 * set + 3 + i]) * (double)cf[6 * set + 3 + j];
-                    const double *o = ing + 8 * set;
+                    const double Ku = set == 0 ? P.k0 : P.k2, Kv = set == 0 ? P.k1 : P.k2;
+                    const double su2 = (Ku * (double)ci[2 * set]) * (double)cj[2 * set];
+                    const double sv2 = (Kv * (double)ci[2 * set + 1]) * (double)cj[2 * set + 1];
+                    const double *o = rec + 8 * set;
                     const double inv = o[6], add = o[7];
                     double lu[3], lv[3];
                     for (int a = 0; a < 3; a++)
@@ -313,17 +384,32 @@ k_assemble_rows(DeviceBatch d)
                     ks[q] = ks[q] + h[q];
             }
             // bending: float(-(l_a g_b)) per edge, edges ascending, negated total
-            for (int it = d.b_ptr[blk]; it < d.b_ptr[blk + 1]; it++)
+            for (int it = e0; it < e1; it += TOGETHER)
             {
-                const int code = d.b_list[it];
-                const int e = code >> 4, i = (code >> 2) & 3, j = code & 3;
-                const double *ing = d.ie_ing + (size_t)ING * e;
-                for (int a = 0; a < 3; a++)
-                    for (int b = 0; b < 3; b++)
+                double l[TOGETHER][3], g[TOGETHER][3];
+#pragma unroll
+                for (int u = 0; u < TOGETHER; u++)
+                {
+                    const double *ing = d.ie_ing + (size_t)ING * (edge[u] >> 4);
+                    const int i = (edge[u] >> 2) & 3, j = edge[u] & 3;
+                    for (int a = 0; a < 3; a++)
                     {
-                        const float hf = (float)(-(ing[3 * i + a] * ing[12 + 3 * j + b]));
-                        kb[3 * a + b] = kb[3 * a + b] + (double)hf;
+                        l[u][a] = ing[3 * i + a];
+                        g[u][a] = ing[12 + 3 * j + a];
                     }
+                }
+#pragma unroll
+                for (int u = 0; u < TOGETHER; u++)
+                    edge[u] = d.b_list[min(it + TOGETHER + u, e1 - 1)];
+#pragma unroll
+                for (int u = 0; u < TOGETHER; u++)
+                    if (it + u < e1)
+                        for (int a = 0; a < 3; a++)
+                            for (int b = 0; b < 3; b++)
+                            {
+                                const float hf = (float)(-(l[u][a] * g[u][b]));
+                                kb[3 * a + b] = kb[3 * a + b] + (double)hf;
+                            }
             }
             for (int q = 0; q < 9; q++)
                 w[q] = P.sk * (ks[q] + (-1 * kb[q]));
@@ -333,9 +419,9 @@ k_assemble_rows(DeviceBatch d)
                 w[0] = mm + w[0];
                 w[4] = mm + w[4];
                 w[8] = mm + w[8];
-                diag[0] = w[0];
-                diag[1] = w[4];
-                diag[2] = w[8];
+                diag[0][lane] = w[0];
+                diag[1][lane] = w[4];
+                diag[2][lane] = w[8];
             }
             if (pin_p || d.row_pinned[c])
                 for (int q = 0; q < 9; q++)
@@ -352,25 +438,9 @@ k_assemble_rows(DeviceBatch d)
             W32[(9 * k + q) * SLICE] = (float)w[q];
         }
     }
-    // force: stretch sum over incident triangles, then bending over incident
-    // interior edges (CalcTotalForce BaraffMaterial.cpp:267-282,
-    // AssignForceAndMatrix DihedralBending.cpp:449-489)
-    double fs[3] = {0.0, 0.0, 0.0}, fb[3] = {0.0, 0.0, 0.0};
-    for (int it = d.vt_ptr[vg]; it < d.vt_ptr[vg + 1]; it++)
-    {
-        const int code = d.vt_list[it];
-        const double *ing = d.tri_ing + (size_t)ING * (code >> 2) + 16 + 3 * (code & 3);
-        for (int a = 0; a < 3; a++)
-            fs[a] = fs[a] + ing[a];
-    }
-    for (int it = d.ve_ptr[vg]; it < d.ve_ptr[vg + 1]; it++)
-    {
-        const int code = d.ve_list[it];
-        const double *ing = d.ie_ing + (size_t)ING * (code >> 2);
-        const int i = code & 3;
-        for (int a = 0; a < 3; a++)
-            fb[a] = fb[a] + (ing[24] * ing[12 + 3 * i + a]) / 2;
-    }
+    __syncthreads();
+    if (!last || !row)
+        return;
     const double dt = P.dt, dt2 = dt * dt;
     const size_t r3 = 3 * (size_t)p;
     for (int a = 0; a < 3; a++)
@@ -385,7 +455,7 @@ k_assemble_rows(DeviceBatch d)
         d.dx[r3 + a] = pin_p ? 0.0 : x - xp;
         if (d.dx32)
             d.dx32[r3 + a] = 0.0f;
-        const double pinv = pin_p ? 0.0 : 1.0 / diag[a];
+        const double pinv = pin_p ? 0.0 : 1.0 / diag[a][lane];
         d.P64[r3 + a] = pinv;
         d.P32[r3 + a] = (float)pinv;
     }
@@ -406,7 +476,7 @@ void launch_elements(const DeviceBatch &d, hipStream_t s)
 
 void launch_assemble_rows(const DeviceBatch &d, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_assemble_rows, dim3(d.n_slices), dim3(SLICE), 0, s, d);
+    hipLaunchKernelGGL(k_assemble_rows, dim3(d.n_slices), dim3(ROW_WAVES * SLICE), 0, s, d);
 }
 
 } // namespace bw

@@ -7,7 +7,7 @@ import pytest
 
 from acousticsim_amd import capi
 from acousticsim_amd import workloads as wl
-from obj_fixture import obj_config
+from obj_fixture import hub_config
 
 pytestmark = pytest.mark.gpu
 
@@ -79,27 +79,11 @@ def test_hub_rows_same_bits(monkeypatch, tmp_path, spokes, precision):
     """a vertex with a spoke to each of a ring: its slice alone is wide, its
     blocks past the registers fit in LDS beside the others' (20, 60 in FP32)
     or are read from memory in part"""
-    n = np.arange(spokes)
-    rings = [[0.02 * k * np.cos(2 * np.pi * n / spokes), 0.02 * k * np.sin(2 * np.pi * n / spokes)]
-             for k in range(1, 5)]
-    xy = np.vstack([np.zeros((1, 2))] + [np.array(r).T for r in rings])
-    tri = [(0, 1 + i, 1 + (i + 1) % spokes) for i in n]
-    for k in range(3):
-        a = 1 + k * spokes
-        for i in n:
-            j = (i + 1) % spokes
-            tri += [(a + i, a + spokes + i, a + j), (a + j, a + spokes + i, a + spokes + j)]
-    path = tmp_path / "hub.obj"
-    path.write_text("".join("v %.9g %.9g 0\n" % tuple(p) for p in xy) +
-                    "".join("vt %.9g %.9g\n" % tuple(0.3 * p) for p in xy) +
-                    "".join("f %d/%d %d/%d %d/%d\n" % tuple(np.repeat(t, 2) + 1) for t in tri))
-    conf = obj_config(path, precision=precision, cloth_obj_translation=[0, 0, 0],
-                      constraints={"static_point": [[-0.08, 0.0], [0.08, 0.0]]})
-    x0 = wl.jitter(np.hstack([xy, np.zeros((len(xy), 1))]), 7)
+    cloth = hub_config(tmp_path / "hub.obj", spokes, precision=precision)
     monkeypatch.setenv("BW_SPMV_LPR", "1")
     monkeypatch.setenv("BW_SPMV_STAGE", "0")
     monkeypatch.setenv("BW_SPMV_NT", "0")
-    _same(*(_run(monkeypatch, [(conf, x0)], 2, r) for r in "10"))
+    _same(*(_run(monkeypatch, [cloth], 2, r) for r in "10"))
 
 
 def test_fp64_matrix_same_bits(monkeypatch):
