@@ -238,10 +238,10 @@ k_bend_elements(int n_ie, const int *__restrict__ ie_rows, const double *__restr
 // (block -> list -> element record, per contribution), 25 us for the
 // diagonal's and 90 with all of a row's slots in one lane, and on a full chip
 // the chains that a CU holds at once.  So the slots run side by side, and a
-// block's lists and records are read ahead of the sums.  One wavefront a
-// slice without that, 8, 14: 5 x 5 vertices 91, 19, 20 us, 257 x 257 286, 206, 165, 600 x
-// 600 (0.5 GB written) 1588, 832, 779, 64 clothes of 256 to 16,384 vertices
-// 1851, 977, 912.
+// block's lists and records are read ahead of the sums.  us a call with one
+// wavefront a slice and nothing read ahead, 8, 14: 5 x 5 vertices 91, 19, 20;
+// 257 x 257 286, 206, 165; 600 x 600 (0.5 GB written) 1588, 832, 779; 64
+// clothes of 17 x 17 to 129 x 129 1851, 977, 912.
 constexpr int ROW_WAVES = 14;
 // Contributions to a block (to a force) whose records are read together: a
 // grid's diagonal block has 12 edges

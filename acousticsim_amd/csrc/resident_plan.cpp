@@ -74,8 +74,8 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
     std::vector<ResidentPart> part;
     std::vector<int> halo_row, rows;
     std::vector<uint16_t> pos(col.size(), 0);
-    // per row: the last part that met it outside its own rows, and its
-    // place in that part's halo
+    // per row: the last part that met it, and its place among that part's
+    // directions (own rows, then the halo)
     std::vector<int> met(d_.n_rows, -1);
     std::vector<uint16_t> place(d_.n_rows, 0);
     int stamp = -1;
@@ -102,10 +102,15 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
                          e1 = slice_off[s - 1] + (size_t)slice_w[s - 1] * SLICE;
             rows.clear();
             stamp++;
+            for (int c = r0; c < r1; c++)
+            {
+                met[c] = stamp;
+                place[c] = (uint16_t)(c - r0);
+            }
             for (size_t e = e0; e < e1; e++)
             {
                 const int c = col[e];
-                if ((c < r0 || c >= r1) && met[c] != stamp)
+                if (met[c] != stamp)
                 {
                     met[c] = stamp;
                     rows.push_back(c);
@@ -119,7 +124,7 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
             for (size_t h = 0; h < rows.size(); h++)
                 place[rows[h]] = (uint16_t)(hold * SLICE + h);
             for (size_t e = e0; e < e1; e++)
-                pos[e] = col[e] >= r0 && col[e] < r1 ? (uint16_t)(col[e] - r0) : place[col[e]];
+                pos[e] = place[col[e]];
             halo_row.insert(halo_row.end(), rows.begin(), rows.end());
             part.push_back(p);
         }
