@@ -546,23 +546,55 @@ k_resident(ResidentLaunch a)
         };
         // the slice's rows of W64 times the vectors v of the LDS array, in
         // the order of the variant with L lanes per row
+        // slots whose blocks are read together: 3 with one lane per row (4
+        // spill), else one by one.  The FP64 matrix comes from memory, a trip
+        // a round: with all iterations on it 257 x 257 26.3 -> 18.5 us an
+        // iteration, 125 x 125 12.4 -> 12.1 (10.3 by launches: there a CU
+        // streams 470 KB an iteration), 21 x 21 9.3 -> 8.3; a 5 x 5 cloth's
+        // step, 7 true residuals, 333 -> 305 us
+        constexpr int C64 = L == 1 ? 3 : 1;
         auto product64 = [&](const auto *v, double (&sum)[3]) {
             double y[3][L] = {};
             const G<uint16_t> *pos = glob(rb.pos) + base + here(lane);
             const G<double> *W64 = glob(d.W64) + 9 * (size_t)base + here(lane);
 #pragma clang loop unroll(disable)
-            for (int k0 = 0; k0 < ws; k0 += L)
+            for (int k0 = 0; k0 < ws; k0 += C64 * L)
+            {
+                if constexpr (C64 == 1)
+                {
 #pragma unroll
-                for (int j = 0; j < L; j++)
-                    if (k0 + j < ws)
+                    for (int j = 0; j < L; j++)
+                        if (k0 + j < ws)
+                        {
+                            const auto *x = v + 3 * (int)pos[(k0 + j) * SLICE];
+                            const G<double> *w = W64 + 9 * (k0 + j) * SLICE;
+                            for (int i = 0; i < 3; i++)
+                                y[i][j] += block<REF>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
+                                                      w[(3 * i + 2) * SLICE], (double)x[0],
+                                                      (double)x[1], (double)x[2]);
+                        }
+                }
+                else
+                {
+                    double w[C64][9];
+                    int at[C64];
+#pragma unroll
+                    for (int c = 0; c < C64; c++)
                     {
-                        const auto *x = v + 3 * (int)pos[(k0 + j) * SLICE];
-                        const G<double> *w = W64 + 9 * (k0 + j) * SLICE;
-                        for (int i = 0; i < 3; i++)
-                            y[i][j] += block<REF>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
-                                                  w[(3 * i + 2) * SLICE], (double)x[0],
-                                                  (double)x[1], (double)x[2]);
+                        const int k = min(k0 + c, ws - 1);
+                        at[c] = 3 * (int)pos[k * SLICE];
+                        for (int q = 0; q < 9; q++)
+                            w[c][q] = W64[(9 * k + q) * SLICE];
                     }
+#pragma unroll
+                    for (int c = 0; c < C64; c++)
+                        if (k0 + c < ws)
+                            for (int i = 0; i < 3; i++)
+                                y[i][0] += block<REF>(w[c][3 * i], w[c][3 * i + 1],
+                                                      w[c][3 * i + 2], (double)v[at[c]],
+                                                      (double)v[at[c] + 1], (double)v[at[c] + 2]);
+                }
+            }
             for (int i = 0; i < 3; i++)
                 sum[i] = phases<L>(y[i]);
         };
