@@ -345,6 +345,9 @@ k_resident(ResidentLaunch a)
     extern __shared__ __align__(16) unsigned char rs_lds[];
     __shared__ int sh_ticket, sh_failed;
     __shared__ CgState sh_st;
+    // REF: the slices' sums of this part, apart from the parts' sums, which
+    // the other wavefronts gather while the first one adds these
+    __shared__ double sh_slices[REF ? 3 * WAVES : 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
     const int E = NT + a.halo_max;
     T *dl = reinterpret_cast<T *>(rs_lds);               // directions, 3 an entry
@@ -489,16 +492,16 @@ k_resident(ResidentLaunch a)
         // store per wavefront; smaller cloths within 4%).
         auto publish = [&](double v, int span, int n, G<u64> *words, double *sm) {
             const int l = here(lane), at = l / span;
-            if (have && at < n && l % span == 0)
-                sm[n * (sl - pt.set0) + at] = v;
             if constexpr (REF)
             {
                 // pcg.hip's block_sum: the wavefronts in order
+                if (have && at < n && l % span == 0)
+                    sh_slices[n * wave + at] = v;
                 __syncthreads();
                 const int t = here(tid);
                 if (t >= 2 * n || (!shared && (t & 1)))
                     return;
-                const double *from = sm + n * (pt.slice0 - pt.set0) + t / 2;
+                const double *from = sh_slices + t / 2;
                 const double sum = ((from[0] + from[n]) + from[2 * n]) + from[3 * n];
                 if (!shared)
                     sm[t / 2] = sum;
@@ -507,6 +510,8 @@ k_resident(ResidentLaunch a)
                                (unsigned)(t & 1 ? __double2hiint(sum) : __double2loint(sum)));
                 return;
             }
+            if (have && at < n && l % span == 0)
+                sm[n * (sl - pt.set0) + at] = v;
             if (!shared)
                 return;
             __syncthreads();

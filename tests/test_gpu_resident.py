@@ -118,8 +118,12 @@ def test_given_up_launch_solves_by_launches(monkeypatch):
           _run(monkeypatch, cloths, 2, "0"))
 
 
+# the last three: clothes of 11, 17 and 66 parts, from where the parts' sums of
+# a true residual, of r.z and r.r, and of d.q reach past the first wavefront's
+# words
 @pytest.mark.parametrize("rows,cols,max_iters", [(2, 2, 20), (9, 9, 1), (9, 9, 2), (16, 16, 90),
-                                                 (17, 16, 90), (33, 70, 150)])
+                                                 (17, 16, 90), (33, 70, 150), (52, 53, 150),
+                                                 (65, 65, 200), (129, 129, 120)])
 def test_reference_semantics_same_bits(monkeypatch, rows, cols, max_iters):
     """the fixed iteration count in one launch against pcg.hip's launches"""
     conf, x0 = _grid(rows, cols, "fp64")
