@@ -33,11 +33,11 @@ class StepStats(ctypes.Structure):
         ("rel_residual", ctypes.c_double),
         ("step_us", ctypes.c_double),
         ("matrix_fp64", ctypes.c_int),
-        ("reserved", ctypes.c_int),
+        ("solve_route", ctypes.c_int),
     ]
 
     def as_dict(self):
-        return {k: getattr(self, k) for k, _ in self._fields_ if k != "reserved"}
+        return {k: getattr(self, k) for k, _ in self._fields_}
 
 
 class RequestInfo(ctypes.Structure):

@@ -1087,7 +1087,7 @@ void Batch::solve_ref(const std::function<void()> &again)
                 pred_launches_.assign(size(), 0);
             for (int i = 0; i < size(); i++)
             {
-                take_stats(i, host_cg_[2 * i]);
+                take_stats(i, host_cg_[2 * i], ROUTE_RESIDENT);
                 stats_[i].outer_iterations = 1;
             }
             return;
@@ -1116,6 +1116,7 @@ void Batch::solve_ref(const std::function<void()> &again)
         StepStats &st = stats_[i];
         st.pcg_iterations = s.total_iter;
         st.outer_iterations = 1;
+        st.solve_route = ROUTE_LAUNCHES;
         st.rel_residual = s.bb > 0 ? std::sqrt(s.rr64 / s.bb) : std::sqrt(s.rr64);
         most = std::max(most, s.total_iter);
     }
@@ -1358,9 +1359,10 @@ bool Batch::lane_update(Lane &L, long long cap)
     return any;
 }
 
-void Batch::take_stats(int i, const CgState &s)
+void Batch::take_stats(int i, const CgState &s, SolveRoute route)
 {
     StepStats &st = stats_[i];
+    st.solve_route = route;
     st.pcg_iterations = s.total;
     st.outer_iterations = s.updates;
     st.matrix_fp64 = s.w64;
@@ -1384,7 +1386,7 @@ void Batch::solve_cg(const std::function<void()> &again)
         {
             solved_[i] = resident_.count[i] > 0;
             if (solved_[i])
-                take_stats(i, host_cg_[2 * i]);
+                take_stats(i, host_cg_[2 * i], ROUTE_RESIDENT);
             all &= solved_[i] != 0;
         }
         if (all)
@@ -1476,7 +1478,7 @@ void Batch::solve_cg(const std::function<void()> &again)
     for (int k = 0; k < nl; k++)
         for (int i : lanes_[k].members)
             if (!solved_[i])
-                take_stats(i, lanes_[k].host_cg[2 * i]);
+                take_stats(i, lanes_[k].host_cg[2 * i], nl > 1 ? ROUTE_LANES : ROUTE_LAUNCHES);
 }
 
 void Batch::begin_step()

@@ -21,6 +21,15 @@ struct StepStats
     double rel_residual = 0;
     double step_us = 0;
     int matrix_fp64 = 0; // mixed form: the last solve moved to the FP64 matrix
+    int solve_route = 0; // SolveRoute of the last solve
+};
+
+// how a cloth's solve ran (bw_step_stats::solve_route)
+enum SolveRoute
+{
+    ROUTE_LAUNCHES = 0, // launches per iteration, one chain
+    ROUTE_LANES = 1,    // the same, in lanes on separate streams
+    ROUTE_RESIDENT = 2  // one launch (resident.h)
 };
 
 // how a batch solves: the reference's own PCG with exactly max_iters-1
@@ -236,7 +245,7 @@ private:
     // (after a one-launch solve that was given up)
     void solve_ref(const std::function<void()> &again);
     void solve_cg(const std::function<void()> &again);
-    void take_stats(int i, const CgState &s);
+    void take_stats(int i, const CgState &s, SolveRoute route);
     // One-launch solves (resident_plan.cpp).  build_resident: the cloths
     // that fit them as parts, given the layout's columns; solve_resident:
     // one launch over those cloths, false when it was given up and all

@@ -54,7 +54,8 @@ typedef struct bw_step_stats
     double step_us;       /* host wall time of the last step */
     int matrix_fp64;      /* "mixed": 1 when the last solve stalled on the FP32
                              matrix and finished on the FP64 one */
-    int reserved;
+    int solve_route;      /* how the last step was solved: 2 one launch, 0 launches
+                             per iteration, 1 launches in a batch's lanes */
 } bw_step_stats;
 
 /* ---- single cloth: the cBaseCloth interface --------------------------- */

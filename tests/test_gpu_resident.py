@@ -41,7 +41,13 @@ def _run(monkeypatch, cloths, steps, resident, **env):
     return out, st
 
 
-def _same(a, b):
+ONE_LAUNCH, LAUNCHES = 2, 0  # solve_route
+
+
+def _same(a, b, route=ONE_LAUNCH):
+    """a's results are b's, a having solved by `route` and b by launches"""
+    assert [s["solve_route"] for s in a[1]] == [route] * len(a[1])
+    assert not any(s["solve_route"] == ONE_LAUNCH for s in b[1])
     for i, (x, y) in enumerate(zip(a[0], b[0])):
         assert np.array_equal(x, y), "cloth %d" % i
     for p, q in zip(a[1], b[1]):
@@ -60,6 +66,17 @@ def test_grid_same_bits(monkeypatch, rows, cols, precision):
     monkeypatch.setenv("BW_SPMV_STAGE", "0")
     monkeypatch.setenv("BW_SPMV_NT", "0")
     _same(_run(monkeypatch, cloth, 2, "1"), _run(monkeypatch, cloth, 2, "0"))
+
+
+# clothes whose sums take several rounds of words and of sets: 352 and 1,000
+# slices (a round: 1,280 words in FP64, 2,560 in the mixed form; 256 sets)
+@pytest.mark.parametrize("rows,cols,precision", [(150, 150, "fp64"), (250, 255, "mixed")])
+def test_large_grid_same_bits(monkeypatch, rows, cols, precision):
+    cloth = [_grid(rows, cols, precision)]
+    monkeypatch.setenv("BW_SPMV_LPR", "1")
+    monkeypatch.setenv("BW_SPMV_STAGE", "0")
+    monkeypatch.setenv("BW_SPMV_NT", "0")
+    _same(*(_run(monkeypatch, cloth, 1, r) for r in "10"))
 
 
 @pytest.mark.parametrize("precision", ["mixed", "fp64"])
@@ -115,7 +132,7 @@ def test_given_up_launch_solves_by_launches(monkeypatch):
     monkeypatch.setenv("BW_SPMV_STAGE", "0")
     monkeypatch.setenv("BW_SPMV_NT", "0")
     _same(_run(monkeypatch, cloths, 2, "1", BW_RESIDENT_GIVE_UP="150"),
-          _run(monkeypatch, cloths, 2, "0"))
+          _run(monkeypatch, cloths, 2, "0"), LAUNCHES)
 
 
 # the last three: clothes of 11, 17 and 66 parts, from where the parts' sums of
@@ -157,4 +174,7 @@ def test_served_same_bits(monkeypatch):
         for rid, x in zip(ids, ref):
             assert s.wait(rid, 60.0) and s.info(rid)["status"] == 0
             assert np.array_equal(s.get_pos(rid), x)
+        # a launch a round, or two an iteration of the stiff cloth's hundreds
+        launches = s.counters()["launches"]
+        assert launches > 500 if give_up != "0" else launches <= 64
         s.close()
