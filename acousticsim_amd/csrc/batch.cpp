@@ -397,7 +397,8 @@ void Batch::build_layout()
         // reliable updates: FP32 recurrences are replaced by the FP64 true
         // residual each time r.r drops by rel2, or after max_since
         // iterations; FP64 recurrences are checked only at convergence.
-        // BW_REL2 and BW_MAX_SINCE override them for tuning runs.
+        // BW_REL2 and BW_MAX_SINCE override them for tuning runs (not with
+        // the reference's semantics, which know no true residual on the way).
         // The forced check's window grows with the cloth's linear size: CG
         // needs iterations in proportion to the mesh's resolution to reduce
         // the residual by a given factor, so a fixed window takes a large
@@ -409,9 +410,9 @@ void Batch::build_layout()
         P.rel2 = mixed ? 1e-2 : 0.0;
         const double side = std::sqrt(std::max(1.0, (double)m.nv / 16384.0));
         P.max_since = mixed ? (int)std::min(2000.0 * side, 1e9) : (1 << 30);
-        if (const char *e = std::getenv("BW_REL2"))
+        if (const char *e = std::getenv("BW_REL2"); e && !P.ref_mode)
             P.rel2 = std::atof(e);
-        if (const char *e = std::getenv("BW_MAX_SINCE"))
+        if (const char *e = std::getenv("BW_MAX_SINCE"); e && !P.ref_mode)
             P.max_since = std::atoi(e);
         // a forced check that finds r.r above 1e-4 of its value at the last
         // replacement (less than 100x down in 2000 iterations) moves the

@@ -150,6 +150,15 @@ def test_reference_semantics_same_bits(monkeypatch, rows, cols, max_iters):
     _same(a, b)
 
 
+def test_reference_semantics_take_no_tuning_window(monkeypatch):
+    """BW_MAX_SINCE forces true residuals in the tolerance modes only"""
+    conf, x0 = _grid(16, 16, "fp64")
+    del conf["precision"]
+    conf.update(solver_mode="reference", max_iters=90)
+    a = _run(monkeypatch, [(conf, x0)], 2, "1", BW_MAX_SINCE="20")
+    _same(a, _run(monkeypatch, [(conf, x0)], 2, "0"))
+
+
 def _reference_mesh(max_iters):
     conf, x0 = _delaunay(700, "fp64")
     del conf["precision"]
