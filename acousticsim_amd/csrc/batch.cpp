@@ -1537,7 +1537,8 @@ void Batch::fixed_variant(int &lpr, int &stage, int &nt) const
 // within 3% of the fastest), timing each on the system assembled at the
 // current state.  BW_SPMV_LPR=1|2|4, BW_SPMV_STAGE=0|1 and
 // BW_SPMV_NT=0|1 in the environment fix those choices instead.
-int Batch::autotune()
+// keep_lpr: of the variants with that many lanes per row (0: any).
+int Batch::autotune(int keep_lpr)
 {
     if (kind_ == SolverKind::RefPCG64 || kind_ == SolverKind::GpuForm)
         return d_.spmv_lpr;
@@ -1545,6 +1546,8 @@ int Batch::autotune()
     tuned_ = true;
     int fixed_lpr = 0, fixed_stage = -1, fixed_nt = -1;
     fixed_variant(fixed_lpr, fixed_stage, fixed_nt);
+    if (keep_lpr)
+        fixed_lpr = keep_lpr;
     double best = 1e300;
     int pick = 0;
     const int choices[3] = {1, 2, 4};
@@ -2350,12 +2353,14 @@ void Batch::step(int nsteps)
         // per row, gathered, cached
         int lpr, stage, nt;
         fixed_variant(lpr, stage, nt);
-        d_.spmv_lpr = lpr ? lpr : 1;
+        d_.spmv_lpr = kept_lpr_ = lpr ? lpr : 1;
         d_.spmv_stage = stage == 1;
         d_.spmv_nt = nt == 1;
     }
     else if (!tuned_)
-        autotune();
+        // after one-launch solves the lanes per row stay: they set the
+        // rounding, and a launch that was given up must not change results
+        autotune(kept_lpr_);
     for (int n = 0; n < nsteps; n++)
     {
         const auto t0 = std::chrono::steady_clock::now();

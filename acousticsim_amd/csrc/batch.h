@@ -117,7 +117,7 @@ public:
     // lanes index (1, 2, 4) + 3 * staged + 6 * nontemporal (0: not timed;
     // the staged form needs every slice to have at most HALO_CAP columns)
     static constexpr int TUNE_VARIANTS = 12;
-    int autotune();
+    int autotune(int keep_lpr = 0);
     // the SpMV choices BW_SPMV_LPR / BW_SPMV_STAGE / BW_SPMV_NT fix (0 / -1:
     // free)
     void fixed_variant(int &lpr, int &stage, int &nt) const;
@@ -291,6 +291,7 @@ private:
     BatchOptions opt_;
     bool own_stream_ = false;
     bool tuned_ = false;
+    int kept_lpr_ = 0; // lanes per row that one-launch solves have followed (0: none yet)
     double tune_us_[TUNE_VARIANTS] = {};
     long long n_halo_ = 0; // entries of the staged SpMV's column lists
     size_t device_bytes_ = 0;

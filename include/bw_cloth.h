@@ -324,7 +324,8 @@ int bw_batch_time_launch_floor(bw_batch *b, int reps, double *avg_us);
    of it, so that near-equal variants do not swap between runs; the first
    bw_batch_step does this by itself when a cloth of the batch solves by
    launches (else it takes 1 lane per row, gathered, cached: the lane count
-   sets the rounding that one-launch solves follow).  A variant is 1, 2 or 4 lanes per matrix row; the
+   sets the rounding that one-launch solves follow, and is kept when the
+   batch falls back to launches).  A variant is 1, 2 or 4 lanes per matrix row; the
    direction vector gathered from memory per slot, or staged in LDS once
    per distinct column of a 64-row slice; matrix loads with or without the
    nontemporal hint.  lanes gets the lanes per row chosen, staged and

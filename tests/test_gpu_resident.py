@@ -135,6 +135,18 @@ def test_given_up_launch_solves_by_launches(monkeypatch):
           _run(monkeypatch, cloths, 2, "0"), LAUNCHES)
 
 
+def test_given_up_launch_keeps_the_rounding(monkeypatch):
+    """the steps after a launch that gave up, whose launches are then tuned,
+    are those of one-launch solves (no variant fixed by the environment: the
+    tuner alone picks 4 lanes for the first cloth and 2 for the second)"""
+    cloths = [_grid(30, 31, "mixed"), _grid(45, 45, "mixed", 5.0)]
+    for cloth in cloths:
+        a = _run(monkeypatch, [cloth], 3, "1", BW_RESIDENT_GIVE_UP="150")
+        b = _run(monkeypatch, [cloth], 3, "1")
+        assert a[1][0]["solve_route"] == LAUNCHES and b[1][0]["solve_route"] == ONE_LAUNCH
+        assert np.array_equal(a[0][0], b[0][0])
+
+
 # the last three: clothes of 11, 17 and 66 parts, from where the parts' sums of
 # a true residual, of r.z and r.r, and of d.q reach past the first wavefront's
 # words
