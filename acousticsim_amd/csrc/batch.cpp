@@ -1567,6 +1567,12 @@ int Batch::autotune(int keep_lpr)
         pick = v;
         candidates++;
     }
+    // timing overwrites the solver states, which carry the choice of matrix
+    // from step to step
+    std::vector<CgState> states(2 * (size_t)size());
+    const size_t state_bytes = states.size() * sizeof(CgState);
+    check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+    check(hipMemcpy(states.data(), d_.cg, state_bytes, hipMemcpyDeviceToHost), "hipMemcpy states");
     if (candidates > 1)
         for (int v = 0; v < TUNE_VARIANTS; v++)
         {
@@ -1586,6 +1592,7 @@ int Batch::autotune(int keep_lpr)
         for (int v = TUNE_VARIANTS - 1; v >= 0; v--)
             if (tune_us_[v] > 0.0 && tune_us_[v] <= 1.03 * best)
                 pick = v;
+    check(hipMemcpy(d_.cg, states.data(), state_bytes, hipMemcpyHostToDevice), "hipMemcpy states");
     set(pick);
     return d_.spmv_lpr;
 }

@@ -135,14 +135,17 @@ def test_given_up_launch_solves_by_launches(monkeypatch):
           _run(monkeypatch, cloths, 2, "0"), LAUNCHES)
 
 
-def test_given_up_launch_keeps_the_rounding(monkeypatch):
+@pytest.mark.parametrize("env", [{}, dict(BW_MAX_SINCE="20", BW_STALL="1e-9")])
+def test_given_up_launch_keeps_the_rounding(monkeypatch, env):
     """the steps after a launch that gave up, whose launches are then tuned,
     are those of one-launch solves (no variant fixed by the environment: the
-    tuner alone picks 4 lanes for the first cloth and 2 for the second)"""
+    tuner alone picks 4 lanes for the first cloth and 2 for the second), also
+    of a cloth that stays on the FP64 matrix from step to step"""
     cloths = [_grid(30, 31, "mixed"), _grid(45, 45, "mixed", 5.0)]
     for cloth in cloths:
-        a = _run(monkeypatch, [cloth], 3, "1", BW_RESIDENT_GIVE_UP="150")
-        b = _run(monkeypatch, [cloth], 3, "1")
+        a = _run(monkeypatch, [cloth], 3, "1", BW_RESIDENT_GIVE_UP="150", **env)
+        b = _run(monkeypatch, [cloth], 3, "1", **env)
+        assert a[1][0]["matrix_fp64"] == b[1][0]["matrix_fp64"] == bool(env)
         assert a[1][0]["solve_route"] == LAUNCHES and b[1][0]["solve_route"] == ONE_LAUNCH
         assert np.array_equal(a[0][0], b[0][0])
 
