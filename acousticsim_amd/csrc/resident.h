@@ -63,7 +63,10 @@ struct ResidentCtl
 {
     int next;     // next ticket
     int aborted;  // 1: a wait ran out; the launch's cloths are not solved
-    int pad[2];
+    int progress; // moves on while any of the launch's cloths does
+    int pad;
+    // of the 100 MHz clock, without a wait's end or progress of any cloth
+    unsigned long long wait_ticks;
 };
 
 struct ResidentLaunch
@@ -77,7 +80,6 @@ struct ResidentLaunch
     int sets_max, halo_max;     // over the launch's parts (halo_max even)
     int extra;                  // slots of slices past RS_SLOTS that a part keeps in LDS
     int give_up;                // tests: abort a cloth after this many iterations (0: never)
-    unsigned long long wait_ticks; // of the 100 MHz clock, per wait
 };
 
 // One such launch at a time on a device: its workgroups wait for one
@@ -86,9 +88,10 @@ struct ResidentLaunch
 std::mutex &resident_turn();
 // slots of slices past RS_SLOTS that a part can keep in LDS, of `wanted`
 int resident_extra(bool fp32, int sets_max, int halo_max, int wanted);
-// when a launch is given up: after a wait of 2 s (BW_RESIDENT_WAIT_MS), or at
-// BW_RESIDENT_GIVE_UP iterations of a cloth (tests)
-void resident_limits(ResidentLaunch &a);
+// when a launch is given up: after a wait of 2 s in which none of its cloths
+// got on (BW_RESIDENT_WAIT_MS), or at BW_RESIDENT_GIVE_UP iterations of a
+// cloth (tests)
+void resident_limits(ResidentLaunch &a, ResidentCtl &ctl);
 // dynamic LDS bytes of a launch
 size_t resident_lds(bool fp32, int sets_max, int halo_max, int extra);
 // workgroups of the launch that are resident at once on the current device

@@ -38,9 +38,10 @@
 // together (resident_capacity; the host checks it) the earliest unfinished
 // cloth has all of its parts running, and the launch ends.  Other work on
 // the device may delay a workgroup, so every wait is bounded all the same
-// (ResidentLaunch::wait_ticks); a wait that runs out sets
-// ResidentCtl::aborted, every workgroup leaves, and the host solves again by
-// launches.
+// (ResidentCtl::wait_ticks, counted while no cloth of the launch gets on: a
+// later cloth's parts may wait through whole solves of earlier ones); a wait
+// that runs out sets ResidentCtl::aborted, every workgroup leaves, and the host
+// solves again by launches.
 //
 // The reference's semantics (solver_mode "reference": FP64, exactly
 // max_iters - 1 iterations, BaraffCloth.cpp:529) are the same recurrences
@@ -98,25 +99,40 @@ template <> struct Pieces<double>
     }
 };
 
-// A bounded wait: true once the time given has passed, or another workgroup
-// has given up (looked at every 64 polls)
+__device__ inline int control(const int *p)
+{
+    return __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
+// A bounded wait: true once the time given has passed without progress
+// anywhere in the launch (a part may wait for a whole solve of the cloths
+// before its own, whose end gives the other parts of its cloth their CUs), or
+// another workgroup has given up (looked at every 64 polls)
 struct Patience
 {
-    u64 ticks;
-    const int *aborted;
+    const ResidentCtl *ctl;
     u64 since;
-    int polls;
+    int polls, seen;
     __device__ bool out()
     {
         if (++polls & 63)
             return false;
         const u64 t = wall_clock64();
-        if (!since)
+        const int now = control(&ctl->next) + control(&ctl->progress);
+        if (!since || now != seen)
+        {
             since = t;
-        return t - since > ticks ||
-               __hip_atomic_load(aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+            seen = now;
+        }
+        return t - since > ctl->wait_ticks || control(&ctl->aborted) != 0;
     }
 };
+// Iterations of an FP64 cloth after which ResidentCtl::progress moves.  A
+// mixed one's moves with every eighth true residual, 33,000 iterations or 0.6 s
+// at most (with every one 5 x 5 and 21 x 21 lost 1.5%, with a test in each
+// iteration 2%).
+constexpr int PROGRESS = 256;
 
 // v, but unknown to the compiler: addresses formed from it are formed where
 // they are used instead of being kept in registers across the solve
@@ -360,7 +376,7 @@ k_resident(ResidentLaunch a)
     T *mx = reinterpret_cast<T *>(hrow + a.halo_max);
     unsigned *cx = reinterpret_cast<unsigned *>(mx + a.extra * 9 * SLICE);
     const int2 *ticket = reinterpret_cast<const int2 *>(a.ctl + 1);
-    const Patience patience = {a.wait_ticks, &a.ctl->aborted, 0, 0};
+    const Patience patience = {a.ctl, 0, 0, 0};
     // every wavefront here, and no wait of the workgroup has run out
     auto meet = [&]() {
         __syncthreads();
@@ -697,7 +713,11 @@ k_resident(ResidentLaunch a)
                 st.w64 = w64;
                 __syncthreads();
                 if (tid == 0)
+                {
                     sh_st = st;
+                    if (pt.slice0 == pt.set0 && (st.updates & 7) == 0)
+                        atomicAdd(&a.ctl->progress, 1);
+                }
                 if (uniform(st.done))
                     break;
                 steps = 0;
@@ -878,6 +898,9 @@ k_resident(ResidentLaunch a)
             rr = t[1];
             steps++;
             first = false;
+            if constexpr (!MIXED)
+                if (steps % PROGRESS == 0 && pt.slice0 == pt.set0 && tid == 0)
+                    atomicAdd(&a.ctl->progress, 1);
             // (NaN and infinity too)
             check = (steps >= room) | (!REF && !(rr > enough && rr < __builtin_inf()));
         }

@@ -50,9 +50,9 @@ int resident_extra(bool fp32, int sets_max, int halo_max, int wanted)
     return std::min(wanted, (int)((RS_LDS_MAX - used) / resident_slot_bytes(fp32)));
 }
 
-void resident_limits(ResidentLaunch &a)
+void resident_limits(ResidentLaunch &a, ResidentCtl &ctl)
 {
-    a.wait_ticks = 100000ULL * (unsigned)std::max(0, env_int("BW_RESIDENT_WAIT_MS", 2000));
+    ctl.wait_ticks = 100000ULL * (unsigned)std::max(0, env_int("BW_RESIDENT_WAIT_MS", 2000));
     a.give_up = env_int("BW_RESIDENT_GIVE_UP", 0);
 }
 
@@ -248,7 +248,7 @@ bool Batch::solve_resident(const std::function<void()> &again)
     a.sets_max = rp.sets_max;
     a.halo_max = rp.halo_max;
     a.extra = extra;
-    resident_limits(a);
+    resident_limits(a, *ctl);
     int aborted = 0;
     {
         std::lock_guard<std::mutex> turn(resident_turn());

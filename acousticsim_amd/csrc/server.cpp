@@ -481,7 +481,7 @@ bool Server::launch_one(std::vector<Resident *> &one, std::unique_lock<std::mute
             *ticket++ = make_int2(r->slot, k);
     a.table = rs_table_dev_;
     a.ctl = reinterpret_cast<ResidentCtl *>(rs_ctl_dev_);
-    resident_limits(a);
+    resident_limits(a, *ctl);
     turn = std::unique_lock<std::mutex>(resident_turn());
     check(hipMemcpyAsync(rs_ctl_dev_, rs_ctl_host_, bytes, hipMemcpyHostToDevice, stream_),
           "hipMemcpyAsync tickets");

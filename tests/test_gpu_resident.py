@@ -124,6 +124,21 @@ def test_more_parts_than_the_chip_holds(monkeypatch):
     _same(_run(monkeypatch, cloths, 1, "1"), _run(monkeypatch, cloths, 1, "0"))
 
 
+@pytest.mark.parametrize("precision,wait_ms", [("mixed", "4"), ("fp64", "8")])
+def test_waiting_for_another_cloth_is_no_lost_wait(monkeypatch, precision, wait_ms):
+    """waits bounded to less than a solve takes: the parts of a cloth that the
+    chip holds only in part wait for the solves before it (with many true
+    residuals: the mixed form's progress is seen at every eighth)"""
+    monkeypatch.setenv("BW_REL2", "0.5" if precision == "mixed" else "0")
+    cloths = [_grid(70 + k, 90, precision, 5.0) for k in range(28)]
+    monkeypatch.setenv("BW_SPMV_LPR", "1")
+    monkeypatch.setenv("BW_SPMV_STAGE", "0")
+    monkeypatch.setenv("BW_SPMV_NT", "0")
+    a = _run(monkeypatch, cloths, 1, "1", BW_RESIDENT_WAIT_MS=wait_ms)
+    assert max(s["pcg_iterations"] for s in a[1]) > 1500
+    _same(a, _run(monkeypatch, cloths, 1, "0"))
+
+
 def test_given_up_launch_solves_by_launches(monkeypatch):
     """a launch that gives up mid-solve (some cloths solved, others not)
     leaves the step to the launches, with their results"""
