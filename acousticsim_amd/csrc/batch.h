@@ -102,14 +102,15 @@ public:
     void end_step(const CgState *states, double step_us);
     // between the two, for a one-cloth batch whose solve one launch may take
     // (resident.h): its parts (0: none), its entry of the launch's table,
-    // what it asks of the launch's LDS, and, after a launch that was given
-    // up, the system and the state of the solve's start again (the batch
-    // has no parts from then on)
+    // what it asks of the launch's LDS, and, when the device cannot hold its
+    // parts, or after a launch that was given up, no parts from then on (after
+    // a launch: with the system and the state of the solve's start again)
     int resident_parts() const { return resident_.given_up ? 0 : resident_.parts; }
     const ResidentBatch &resident_entry() const { return resident_.entry; }
     int resident_sets() const { return resident_.sets_max; }
     int resident_halo() const { return resident_.halo_max; }
     int resident_extra_slots() const { return resident_.extra; }
+    void drop_parts() { resident_.given_up = true; }
     void restart_step();
     size_t device_bytes() const { return device_bytes_; }
     // choose the SpMV variant by timing (done by the first step()); returns

@@ -79,6 +79,9 @@ struct ResidentLaunch
     int lpr;
     int sets_max, halo_max;     // over the launch's parts (halo_max even)
     int extra;                  // slots of slices past RS_SLOTS that a part keeps in LDS
+    // iterations of a cloth after which its solve pauses until the next launch
+    // (0: never); only with one lane per row
+    int pause;
     int give_up;                // tests: abort a cloth after this many iterations (0: never)
 };
 
@@ -96,7 +99,7 @@ void resident_limits(ResidentLaunch &a, ResidentCtl &ctl);
 size_t resident_lds(bool fp32, int sets_max, int halo_max, int extra);
 // workgroups of the launch that are resident at once on the current device
 // (0 when the kernel cannot run with that LDS)
-int resident_capacity(bool fp32, int lpr, size_t lds);
+int resident_capacity(bool fp32, int lpr, size_t lds, bool pause = false);
 void launch_resident(const ResidentLaunch &a, bool fp32, int grid, hipStream_t s);
 // solver states of a solve that is started again (after an aborted launch):
 // the solve start, with the history that k_cg_reset had given it

@@ -434,27 +434,64 @@ void Server::retire(Resident &r, int error_code, const std::string &error)
     cv_budget_.notify_all();
 }
 
+// The launches (two an iteration) that a request's step is expected to need
+// yet: as many as the step before; in a first step of a one-launch solve, 12
+// iterations a vertex of the cloth's side (9 to 16 in the measured cases); a
+// quarter more where that has proved too few.
+long long Server::expected(const Resident &r) const
+{
+    const bool one = r.batch->resident_parts() > 0;
+    long long need = r.predicted;
+    if (need == 0 && one)
+        need = (long long)(24.0 * std::sqrt((double)r.batch->model(0).nv));
+    if (need > r.launched)
+        return need - r.launched;
+    return one ? std::max(64LL, r.launched / 4) : 64LL;
+}
+
 // One launch takes the current step's solve of every request whose cloth
 // fits: the most iterations first (by the step before; in a first step the
 // largest cloth), since the launch lasts as long as its last cloth.
-bool Server::launch_one(std::vector<Resident *> &one, std::unique_lock<std::mutex> &turn)
+void Server::launch_one(std::vector<Resident *> &one, std::vector<Resident *> &many,
+                        long long want, std::unique_lock<std::mutex> &turn)
 {
     ResidentLaunch a = {};
-    int most = 0, extra = 0;
-    for (Resident *r : one)
+    int most = 0, capacity = 0;
+    for (;;)
     {
-        a.tickets += r->batch->resident_parts();
-        most = std::max(most, r->batch->resident_parts());
-        a.sets_max = std::max(a.sets_max, r->batch->resident_sets());
-        a.halo_max = std::max(a.halo_max, r->batch->resident_halo());
-        extra = std::max(extra, r->batch->resident_extra_slots());
+        int extra = 0;
+        a = ResidentLaunch();
+        most = 0;
+        for (Resident *r : one)
+        {
+            a.tickets += r->batch->resident_parts();
+            most = std::max(most, r->batch->resident_parts());
+            a.sets_max = std::max(a.sets_max, r->batch->resident_sets());
+            a.halo_max = std::max(a.halo_max, r->batch->resident_halo());
+            extra = std::max(extra, r->batch->resident_extra_slots());
+        }
+        a.lpr = opt_.spmv_lpr;
+        a.extra = resident_extra(opt_.fp32, a.sets_max, a.halo_max, extra);
+        capacity = resident_capacity(
+            opt_.fp32, a.lpr, resident_lds(opt_.fp32, a.sets_max, a.halo_max, a.extra), true);
+        if (most <= capacity)
+            break;
+        for (Resident *r : one)
+            if (r->batch->resident_parts() > capacity)
+            {
+                r->batch->drop_parts();
+                many.push_back(r);
+            }
+        one.erase(std::remove_if(one.begin(), one.end(),
+                                 [](Resident *r) { return r->batch->resident_parts() == 0; }),
+                  one.end());
     }
-    a.lpr = opt_.spmv_lpr;
-    a.extra = resident_extra(opt_.fp32, a.sets_max, a.halo_max, extra);
-    const int capacity = resident_capacity(
-        opt_.fp32, a.lpr, resident_lds(opt_.fp32, a.sets_max, a.halo_max, a.extra));
-    if (capacity < most)
-        return false;
+    if (one.empty())
+        return;
+    // (at most 2048 iterations, some 20 ms, which a new request may have to wait)
+    a.pause = (int)std::min(2048LL, want / 2);
+    if (const char *e = std::getenv("BW_RESIDENT_PAUSE")) // tests
+        a.pause = std::max(1, std::atoi(e));
     const size_t bytes = sizeof(ResidentCtl) + (size_t)a.tickets * sizeof(int2);
     if (bytes > rs_ctl_cap_)
     {
@@ -492,11 +529,10 @@ bool Server::launch_one(std::vector<Resident *> &one, std::unique_lock<std::mute
     check(hipMemcpyAsync(rs_ctl_host_, rs_ctl_dev_, sizeof(ResidentCtl), hipMemcpyDeviceToHost,
                          stream_),
           "hipMemcpyAsync control");
-    return true;
 }
 
 // One chunk of launches over the requests `many`; its length.
-int Server::run_many(const std::vector<Resident *> &many)
+int Server::run_many(const std::vector<Resident *> &many, long long want)
 {
     // lists of their slices and solver workgroups
     int n = 0, nb = 0, ng = 0;
@@ -566,10 +602,6 @@ int Server::run_many(const std::vector<Resident *> &many)
     check(hipMemcpyAsync(upd_list_dev_, upd_list_host_, ugrid * sizeof(int2),
                          hipMemcpyHostToDevice, stream_),
           "hipMemcpyAsync list");
-    // run until the request expected to finish first should be done
-    long long want = 1LL << 40;
-    for (Resident *r : many)
-        want = std::min(want, r->predicted > r->launched ? r->predicted - r->launched : 64LL);
     const int length = (int)std::min<long long>(1024, std::max<long long>(32, (want + 31) / 32 * 32));
     run_chunk(length, grid, ggrid);
     for (Resident *r : many)
@@ -598,15 +630,26 @@ int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
     std::vector<Resident *> one, many;
     for (auto &r : res)
         (r->batch->resident_parts() > 0 ? one : many).push_back(r.get());
+    // The round lasts twice as long as the request expected to finish its step
+    // first should need, so that none waits for a much longer one's solve, but
+    // 256 iterations at least, since each round costs some 0.15 ms and a share
+    // of the chip stands idle at its end.  Beside a 257 x 257 cloth a 9 x 9 one
+    // takes 2.5 ms a step and a 33 x 33 one 10 (76 and 114 when a round lasted
+    // as long as its longest solve, 3.1 and 12.4 by launches alone); a
+    // saturated mix of up to 200,000 vertices runs 60.4 cloth-steps/s (61.5
+    // with rounds of whole solves, 49 by launches).
+    long long want = 1LL << 40, want_many = 1LL << 40;
+    for (auto &r : res)
+        want = std::min(want, expected(*r));
+    want = std::max(512LL, 2 * want);
     std::unique_lock<std::mutex> turn;
-    if (!one.empty() && !launch_one(one, turn))
-    {
-        many.insert(many.end(), one.begin(), one.end());
-        one.clear();
-    }
+    if (!one.empty())
+        launch_one(one, many, want, turn);
+    for (Resident *r : many)
+        want_many = std::min(want_many, expected(*r));
     int length = 0;
     if (!many.empty())
-        length = run_many(many);
+        length = run_many(many, std::min(want, want_many));
     // every slot's states in one copy
     int top = 0;
     for (auto &r : res)
@@ -630,6 +673,7 @@ int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
         {
             r->batch->restart_step();
             states_host_[2 * r->slot].done = 0;
+            r->launched = 0;
         }
     }
     // finish the steps whose solve is done
@@ -637,6 +681,11 @@ int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
     for (auto &r : res)
     {
         const CgState &st = states_host_[2 * r->slot];
+        if (!st.done && r->batch->resident_parts() > 0)
+        {
+            r->launched = 2LL * (st.total + st.since + st.updates);
+            continue;
+        }
         if (!st.done)
         {
             const long long cap = 4LL * r->batch->model(0).cfg.solver_max_iters + 64;

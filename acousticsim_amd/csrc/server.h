@@ -108,7 +108,8 @@ private:
         std::unique_ptr<Batch> batch;
         int nsteps = 0, steps_done = 0;
         bool solving = false;
-        long long launched = 0;   // solver launches this step
+        long long launched = 0;   // solver launches this step (or, in one
+                                  // launch, as many as its iterations would take)
         long long predicted = 0;  // launches the previous step needed
         double t_step0 = 0;
     };
@@ -116,7 +117,8 @@ private:
     void builder_loop();
     void device_loop();
     int run_round(std::vector<std::unique_ptr<Resident>> &res);
-    int run_many(const std::vector<Resident *> &many);
+    long long expected(const Resident &r) const;
+    int run_many(const std::vector<Resident *> &many, long long want);
     // final positions to the host (when error_code is BW_OK), device memory
     // and slot back, waiters woken
     void retire(Resident &r, int error_code, const std::string &error);
@@ -131,9 +133,11 @@ private:
     ResidentBatch *rs_table_dev_ = nullptr, *rs_table_host_ = nullptr;
     char *rs_ctl_dev_ = nullptr, *rs_ctl_host_ = nullptr;
     size_t rs_ctl_cap_ = 0;
-    // the launch for the requests `one`, its turn taken by `turn`; false
-    // when the device cannot hold one of them
-    bool launch_one(std::vector<Resident *> &one, std::unique_lock<std::mutex> &turn);
+    // the launch for the requests `one`, its turn taken by `turn`, in which a
+    // solve pauses after `want` launches' worth of iterations; those that the
+    // device cannot hold go over to `many`
+    void launch_one(std::vector<Resident *> &one, std::vector<Resident *> &many, long long want,
+                    std::unique_lock<std::mutex> &turn);
 
     // device tables
     CgState *states_dev_ = nullptr, *states_host_ = nullptr; // 2 per slot

@@ -196,24 +196,61 @@ def _reference_mesh(max_iters):
     return conf, x0
 
 
-def test_served_same_bits(monkeypatch):
-    """requests solved together in one launch a round, also after a launch
-    that gives up mid-solve, against the batch's solver launches"""
-    cloths = [_grid(9, 9, "mixed", 0.2), _delaunay(1200, "mixed"), _grid(45, 45, "mixed", 5.0),
-              _grid(30, 31, "mixed")]
+# pause: iterations after which a round's solves are interrupted; env: a
+# cloth on the FP64 matrix, and many true residuals
+@pytest.mark.parametrize("precision,pause,env", [
+    ("mixed", "", {}), ("mixed", "37", {}), ("fp64", "", {}), ("fp64", "37", {}),
+    ("mixed", "1", dict(BW_REL2="0.3")), ("mixed", "13", dict(BW_MAX_SINCE="20", BW_STALL="1e-9"))])
+def test_served_same_bits(monkeypatch, precision, pause, env):
+    """requests solved together in one launch a round, solves that pause between
+    rounds among them, also after a launch that gives up mid-solve, against the
+    batch's solver launches"""
+    cloths = [_grid(9, 9, precision, 0.2), _delaunay(1200, precision),
+              _grid(45, 45, precision, 5.0), _grid(30, 31, precision)]
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    if pause:
+        monkeypatch.setenv("BW_RESIDENT_PAUSE", pause)
     monkeypatch.setenv("BW_SPMV_LPR", "1")
     monkeypatch.setenv("BW_SPMV_STAGE", "0")
     monkeypatch.setenv("BW_SPMV_NT", "0")
     ref = _run(monkeypatch, cloths, 2, "0")[0]
     monkeypatch.setenv("BW_RESIDENT", "1")
-    for give_up in ("0", "150"):
+    # (a launch is given up at a true residual: an FP64 solve's only one ends it)
+    for give_up in ("0", "150") if precision == "mixed" else ("0",):
         monkeypatch.setenv("BW_RESIDENT_GIVE_UP", give_up)
-        s = capi.Server(budget_bytes=2e9, max_resident=8, precision="mixed")
+        s = capi.Server(budget_bytes=2e9, max_resident=8, precision=precision)
         ids = [s.submit(c, x, 2) for c, x in cloths]
         for rid, x in zip(ids, ref):
             assert s.wait(rid, 60.0) and s.info(rid)["status"] == 0
             assert np.array_equal(s.get_pos(rid), x)
         # a launch a round, or two an iteration of the stiff cloth's hundreds
+        iterations = max(s.info(rid)["pcg_iterations"] for rid in ids)
         launches = s.counters()["launches"]
-        assert launches > 500 if give_up != "0" else launches <= 64
+        if give_up != "0":
+            assert launches > iterations > 500
+        elif pause:
+            # (a true residual where a pause is due lets one iteration pass)
+            assert iterations // (int(pause) + 1) <= launches < iterations // int(pause) + 100
+        else:
+            assert launches <= 64
         s.close()
+
+
+@pytest.mark.parametrize("precision", ["mixed", "fp64"])
+def test_served_short_solves_do_not_wait_for_long_ones(precision):
+    """20 steps of a 9 x 9 cloth beside a stiff 129 x 129 one whose step takes
+    as long: they end within its first steps, not with its 20th"""
+    long, x = _grid(129, 129, precision, 10.0)
+    short, xs = _grid(9, 9, precision)
+    s = capi.Server(budget_bytes=4e9, max_resident=4, precision=precision)
+    warm = s.submit(short, xs, 1)
+    assert s.wait(warm, 60.0)
+    a = s.submit(long, x, 25)
+    while s.info(a)["steps_done"] < 1:
+        assert not s.wait(a, 0.002)
+    b = s.submit(short, xs, 20)
+    assert s.wait(b, 60.0) and s.info(b)["status"] == 0
+    assert s.info(a)["steps_done"] < 12
+    assert s.wait(a, 60.0) and s.info(a)["status"] == 0
+    s.close()
