@@ -1,8 +1,6 @@
 // One-launch tolerance solves (resident.hip): the device layout of a batch's
 // cloths as parts, one workgroup each, and the launcher.
 #pragma once
-#include <mutex>
-
 #include "device.h"
 
 namespace bw
@@ -85,10 +83,28 @@ struct ResidentLaunch
     int give_up;                // tests: abort a cloth after this many iterations (0: never)
 };
 
-// One such launch at a time on a device: its workgroups wait for one
-// another, so two launches that each held part of the chip would both wait.
-// Held from the launch until it has ended.
-std::mutex &resident_turn();
+// The workgroups of a cloth of several parts wait for one another, so two
+// launches that each held part of the chip would both wait.  Launches with such
+// clothes take a seat a workgroup, from the launch until it has ended, and
+// together no more than the device has CUs, so that each has all of its
+// workgroups running whatever CUs the others' are on; a launch whose clothes
+// have one part each waits for nothing and takes none.  First come, first
+// served; a launch with more workgroups than CUs takes them all.
+class ResidentSeats
+{
+public:
+    ResidentSeats() = default;
+    ResidentSeats(const ResidentSeats &) = delete;
+    ResidentSeats &operator=(const ResidentSeats &) = delete;
+    ~ResidentSeats() { give(); }
+    void take(int n); // on the current device; waits
+    void give();      // all that were taken
+
+private:
+    struct Device;
+    Device *of_ = nullptr;
+    int n_ = 0;
+};
 // slots of slices past RS_SLOTS that a part can keep in LDS, of `wanted`
 int resident_extra(bool fp32, int sets_max, int halo_max, int wanted);
 // when a launch is given up: after a wait of 2 s in which none of its cloths

@@ -1,6 +1,7 @@
 // The host side of the one-launch tolerance solve (resident.hip): which
 // cloths of a batch it takes, their parts, and the launch.
 #include <algorithm>
+#include <condition_variable>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -36,12 +37,42 @@ constexpr int ITER_CAP = 1000000;
 
 } // namespace
 
-std::mutex &resident_turn()
+struct ResidentSeats::Device
 {
-    static std::mutex turn[64];
+    std::mutex mu;
+    std::condition_variable cv;
+    int cus = 0, used = 0;
+    long long next = 0, serving = 0; // the queue
+};
+
+void ResidentSeats::take(int n)
+{
+    static Device devices[64];
     int dev = 0;
     check(hipGetDevice(&dev), "hipGetDevice");
-    return turn[dev & 63];
+    Device &d = devices[dev & 63];
+    std::unique_lock<std::mutex> lk(d.mu);
+    if (d.cus == 0)
+        check(hipDeviceGetAttribute(&d.cus, hipDeviceAttributeMultiprocessorCount, dev),
+              "hipDeviceGetAttribute");
+    n = std::min(n, d.cus);
+    const long long place = d.next++;
+    d.cv.wait(lk, [&] { return d.serving == place && d.used + n <= d.cus; });
+    d.serving++;
+    d.used += n;
+    of_ = &d;
+    n_ = n;
+    d.cv.notify_all(); // the next in the queue may fit too
+}
+
+void ResidentSeats::give()
+{
+    if (!of_)
+        return;
+    std::lock_guard<std::mutex> lk(of_->mu);
+    of_->used -= n_;
+    of_->cv.notify_all();
+    of_ = nullptr;
 }
 
 int resident_extra(bool fp32, int sets_max, int halo_max, int wanted)
@@ -251,12 +282,15 @@ bool Batch::solve_resident(const std::function<void()> &again)
     resident_limits(a, *ctl);
     int aborted = 0;
     {
-        std::lock_guard<std::mutex> turn(resident_turn());
+        const int grid = std::min(rp.parts, rp.capacity);
+        ResidentSeats seats;
+        if (rp.most > 1)
+            seats.take(grid);
         check(hipMemcpyAsync(rp.ctl, rp.host_ctl,
                              sizeof(ResidentCtl) + (size_t)rp.parts * sizeof(int2),
                              hipMemcpyHostToDevice, stream_),
               "hipMemcpyAsync tickets");
-        launch_resident(a, fp32, std::min(rp.parts, rp.capacity), stream_);
+        launch_resident(a, fp32, grid, stream_);
         check(hipGetLastError(), "resident launch");
         check(hipMemcpyAsync(rp.host_ctl, rp.ctl, sizeof(ResidentCtl), hipMemcpyDeviceToHost,
                              stream_),

@@ -75,6 +75,7 @@ Server::Server(const ServerOptions &opt) : opt_(opt), t0_(std::chrono::steady_cl
           "hipMalloc");
     check(hipHostMalloc((void **)&rs_table_host_, opt_.max_resident * sizeof(ResidentBatch)),
           "hipHostMalloc");
+    check(hipEventCreateWithFlags(&rs_ended_, hipEventDisableTiming), "hipEventCreate");
     check(hipMemset(states_dev_, 0, ns * sizeof(CgState)), "hipMemset");
     check(hipStreamSynchronize(nullptr), "hipStreamSynchronize"); // before the server stream
     for (int s = opt_.max_resident - 1; s >= 0; s--)
@@ -105,6 +106,7 @@ Server::~Server()
     (void)hipStreamSynchronize(stream_);
     (void)hipFree(states_dev_);
     (void)hipFree(table_dev_);
+    (void)hipEventDestroy(rs_ended_);
     (void)hipFree(rs_table_dev_);
     (void)hipHostFree(rs_table_host_);
     (void)hipFree(rs_ctl_dev_);
@@ -453,7 +455,7 @@ long long Server::expected(const Resident &r) const
 // fits: the most iterations first (by the step before; in a first step the
 // largest cloth), since the launch lasts as long as its last cloth.
 void Server::launch_one(std::vector<Resident *> &one, std::vector<Resident *> &many,
-                        long long want, std::unique_lock<std::mutex> &turn)
+                        long long want, ResidentSeats &seats)
 {
     ResidentLaunch a = {};
     int most = 0, capacity = 0;
@@ -519,16 +521,18 @@ void Server::launch_one(std::vector<Resident *> &one, std::vector<Resident *> &m
     a.table = rs_table_dev_;
     a.ctl = reinterpret_cast<ResidentCtl *>(rs_ctl_dev_);
     resident_limits(a, *ctl);
-    turn = std::unique_lock<std::mutex>(resident_turn());
+    // (a sixteenth of the chip stays free for the builders' copies and fills)
+    const int grid = std::min(a.tickets, std::max(most, capacity - capacity / 16));
+    if (most > 1)
+        seats.take(grid);
     check(hipMemcpyAsync(rs_ctl_dev_, rs_ctl_host_, bytes, hipMemcpyHostToDevice, stream_),
           "hipMemcpyAsync tickets");
-    // (a sixteenth of the chip stays free for the builders' copies and fills)
-    launch_resident(a, opt_.fp32, std::min(a.tickets, std::max(most, capacity - capacity / 16)),
-                    stream_);
+    launch_resident(a, opt_.fp32, grid, stream_);
     check(hipGetLastError(), "resident launch");
     check(hipMemcpyAsync(rs_ctl_host_, rs_ctl_dev_, sizeof(ResidentCtl), hipMemcpyDeviceToHost,
                          stream_),
           "hipMemcpyAsync control");
+    check(hipEventRecord(rs_ended_, stream_), "hipEventRecord");
 }
 
 // One chunk of launches over the requests `many`; its length.
@@ -642,9 +646,9 @@ int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
     for (auto &r : res)
         want = std::min(want, expected(*r));
     want = std::max(512LL, 2 * want);
-    std::unique_lock<std::mutex> turn;
+    ResidentSeats seats;
     if (!one.empty())
-        launch_one(one, many, want, turn);
+        launch_one(one, many, want, seats);
     for (Resident *r : many)
         want_many = std::min(want_many, expected(*r));
     int length = 0;
@@ -657,9 +661,10 @@ int Server::run_round(std::vector<std::unique_ptr<Resident>> &res)
     check(hipMemcpyAsync(states_host_, states_dev_, 2 * (size_t)top * sizeof(CgState),
                          hipMemcpyDeviceToHost, stream_),
           "hipMemcpyAsync states");
+    if (!one.empty())
+        check(hipEventSynchronize(rs_ended_), "hipEventSynchronize");
+    seats.give(); // (the launches behind need none)
     check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-    if (turn.owns_lock())
-        turn.unlock();
     {
         std::lock_guard<std::mutex> lk(mu_);
         counters_.chunks += (one.empty() ? 0 : 1) + (many.empty() ? 0 : 1);

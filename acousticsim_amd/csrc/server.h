@@ -133,11 +133,12 @@ private:
     ResidentBatch *rs_table_dev_ = nullptr, *rs_table_host_ = nullptr;
     char *rs_ctl_dev_ = nullptr, *rs_ctl_host_ = nullptr;
     size_t rs_ctl_cap_ = 0;
-    // the launch for the requests `one`, its turn taken by `turn`, in which a
+    hipEvent_t rs_ended_ = nullptr; // that launch
+    // the launch for the requests `one`, its seats taken by `seats`, in which a
     // solve pauses after `want` launches' worth of iterations; those that the
     // device cannot hold go over to `many`
     void launch_one(std::vector<Resident *> &one, std::vector<Resident *> &many, long long want,
-                    std::unique_lock<std::mutex> &turn);
+                    ResidentSeats &seats);
 
     // device tables
     CgState *states_dev_ = nullptr, *states_host_ = nullptr; // 2 per slot

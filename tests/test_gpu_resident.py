@@ -2,6 +2,8 @@
 bits, for cloths of one part and of many, rows narrower and wider than the
 registers hold, both precisions, every lane count whose rounding they follow,
 and after a launch that gives up."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -137,6 +139,38 @@ def test_waiting_for_another_cloth_is_no_lost_wait(monkeypatch, precision, wait_
     a = _run(monkeypatch, cloths, 1, "1", BW_RESIDENT_WAIT_MS=wait_ms)
     assert max(s["pcg_iterations"] for s in a[1]) > 1500
     _same(a, _run(monkeypatch, cloths, 1, "0"))
+
+
+def test_batches_of_several_threads_step_side_by_side():
+    """a cloth of one part does not wait for another thread's long solves, and
+    clothes of several parts, together more than the chip holds, give the
+    results that they give alone"""
+    def batch(cloth):
+        return capi.ClothBatch([cloth[0]], [cloth[1]])
+    big = [_grid(129 + 9 * k, 129, "mixed", 5.0) for k in range(3)] + [_grid(200, 200, "mixed")]
+    alone = []
+    for cloth in big:
+        b = batch(cloth)
+        b.step(4)
+        alone.append(b.get_pos(0))
+        b.close()
+    batches = [batch(c) for c in big]
+    small = batch(_grid(21, 21, "mixed"))
+    small.step(1)
+    threads = [threading.Thread(target=b.step, args=(4,)) for b in batches]
+    for t in threads:
+        t.start()
+    steps = 0
+    while any(t.is_alive() for t in threads):
+        small.step(1)
+        steps += 1
+    for t in threads:
+        t.join()
+    for b, x in zip(batches, alone):
+        assert np.array_equal(b.get_pos(0), x) and b.stats(0)["solve_route"] == ONE_LAUNCH
+    assert small.stats(0)["solve_route"] == ONE_LAUNCH
+    # 16 solves of some 10 ms and more, and steps of 1 ms beside them
+    assert steps > 3 * 16
 
 
 def test_given_up_launch_solves_by_launches(monkeypatch):
