@@ -77,10 +77,10 @@ struct ResidentLaunch
     int lpr;
     int sets_max, halo_max;     // over the launch's parts (halo_max even)
     int extra;                  // slots of slices past RS_SLOTS that a part keeps in LDS
+    int give_up;                // tests: abort a cloth after this many iterations (0: never)
     // iterations of a cloth after which its solve pauses until the next launch
     // (0: never); only with one lane per row
     int pause;
-    int give_up;                // tests: abort a cloth after this many iterations (0: never)
 };
 
 // The workgroups of a cloth of several parts wait for one another, so two

@@ -52,9 +52,8 @@
 //
 // PAUSE, for the server's rounds: after a number of iterations a solve leaves
 // the launch (the recurrences' vectors and scalars to memory), so that a short
-// request need not wait for a long one's solve, and the next launch goes on
-// from the sums of its last iteration, formed again, as if nothing had been
-// between.
+// request need not wait for a long one's solve, and the next launch goes on as
+// if nothing had been between.
 //
 // Same rounding as cg.hip: a row's slots are added per lane phase of the
 // variant with L lanes per row, then the phases; a slice's partial sums in
@@ -365,7 +364,8 @@ k_resident(ResidentLaunch a)
     constexpr int NP = Pieces<T>::N;
     constexpr bool MIXED = sizeof(T) == sizeof(float);
     extern __shared__ __align__(16) unsigned char rs_lds[];
-    __shared__ int sh_ticket, sh_failed, sh_stop;
+    __shared__ int sh_ticket, sh_failed;
+    __shared__ int sh_stop; // PAUSE: iterations of the solve at which it pauses
     __shared__ CgState sh_st;
     // REF: the slices' sums of this part, apart from the parts' sums, which
     // the other wavefronts gather while the first one adds these
@@ -409,25 +409,18 @@ k_resident(ResidentLaunch a)
         // to date at each true residual, in LDS; in between, an iteration
         // needs these scalars only.
         if (tid == 0)
-        {
-            const CgState st = load_state(glob(d.cg) + 2 * inst);
-            sh_st = st;
-            // iterations of the solve at which it pauses
-            sh_stop = PAUSE ? st.total + (st.start ? 0 : st.since) + a.pause : 0;
-        }
+            sh_st = load_state(glob(d.cg) + 2 * inst);
         __syncthreads();
         if (sh_st.done)
             continue;
-        // a solve that has paused starts with the end of its last iteration
-        bool again = PAUSE && uniform(sh_st.start) == 0;
-        bool due = !again;   // PAUSE: a true residual is, whatever the counts
         int steps = 0;       // iterations since the last true residual
         int room = 0;        // after which the next is due
         double enough = 0.0; // r.r at which it is due
         double rho = 0.0;    // r.(P r) of the current direction
         bool first = true;   // the next direction is P r
         bool w64 = uniform(sh_st.w64) != 0;
-        bool check = !again; // a true residual is due (the warm start's)
+        bool check = true;   // a true residual is due (the warm start's)
+        bool due = true;     // PAUSE: whatever the counts
         // sets of sums: one a slice, or one a part
         const int sets = REF ? pt.parts : pt.sets;
         const int set_base = REF ? pt.set0 / BW_SB : pt.set0;
@@ -490,28 +483,6 @@ k_resident(ResidentLaunch a)
         for (int i = tid; i < pt.halo_n; i += NT)
             hrow[i] = rb.halo_row[pt.halo_off + i];
         __syncthreads();
-        if constexpr (PAUSE)
-            if (again)
-            {
-                steps = uniform(sh_st.since);
-                rho = uniform(sh_st.rho);
-                first = false;
-                const G<T> *dp = glob(Vecs<T>::d0(d));
-                for (int i = 0; i < 3; i++)
-                {
-                    r[i] = have ? glob(Vecs<T>::r(d))[3 * row() + i] : (T)0;
-                    dv[i] = have ? dp[3 * row() + i] : (T)0;
-                    if (MIXED)
-                        x32[i] = have ? glob(d.dx32)[3 * row() + i] : 0.0f;
-                }
-                for (int e = tid; e < pt.halo_n; e += NT)
-                    for (int i = 0; i < 3; i++)
-                        dl[3 * (NT + e) + i] = dp[3 * hrow[e] + i];
-                const G<InstParams> *ip = glob(d.params) + inst;
-                room = uniform(min(min(ip->max_iter - sh_st.total, ip->max_since),
-                                   sh_stop - sh_st.total));
-                enough = uniform(fmax(ip->tol * ip->tol * sh_st.bb, ip->rel2 * sh_st.rr_ref));
-            }
 
         // exchange words; those of rows are planes, one per component and
         // piece
@@ -656,6 +627,48 @@ k_resident(ResidentLaunch a)
                 sum[i] = phases<L>(y[i]);
         };
 
+        if constexpr (PAUSE)
+        {
+            const CgState &st = sh_st;
+            if (tid == 0)
+                sh_stop = st.total + (st.start ? 0 : st.since) + a.pause;
+            __syncthreads();
+            if (uniform(st.start) == 0)
+            {
+                // on from where an earlier launch left the solve (below); the
+                // state holds r.z in rr_true's place
+                check = due = first = false;
+                steps = uniform(st.since);
+                rho = uniform(st.rho);
+                rz = uniform(st.rr_true);
+                rr = uniform(st.rr);
+                const G<InstParams> *ip = glob(d.params) + inst;
+                room = uniform(min(min(ip->max_iter - st.total, ip->max_since),
+                                   sh_stop - st.total));
+                enough = uniform(fmax(ip->tol * ip->tol * st.bb, ip->rel2 * st.rr_ref));
+                const G<T> *dp = glob(Vecs<T>::d0(d));
+                for (int i = 0; i < 3; i++)
+                {
+                    r[i] = have ? glob(Vecs<T>::r(d))[3 * row() + i] : (T)0;
+                    dv[i] = have ? dp[3 * row() + i] : (T)0;
+                    if constexpr (MIXED)
+                        x32[i] = have ? glob(d.dx32)[3 * row() + i] : 0.0f;
+                    z[i] = P[i] * r[i];
+                }
+                for (int e = tid; e < pt.halo_n; e += NT)
+                    for (int i = 0; i < 3; i++)
+                        dl[3 * (NT + e) + i] = dp[3 * hrow[e] + i];
+                ++tag;
+                publish_z();
+                // (the other halo entries' z are awaited where they are used)
+                const int e = here(tid);
+                if ((e & ~63) < pt.halo_n &&
+                    !await<3 * NP>(hz, z_tag, patience,
+                                   [&](int w) { return halo_word(words_z, e, w); }))
+                    sh_failed = 1;
+            }
+        }
+
         bool failed = false, paused = false;
         for (;;)
         {
@@ -777,163 +790,155 @@ k_resident(ResidentLaunch a)
                     break;
                 }
             }
-            if (!PAUSE || !again)
+            const double beta = first ? 0.0 : uniform(rz / rho);
+            if (REF && !first && beta == 0.0)
             {
-                const double beta = first ? 0.0 : uniform(rz / rho);
-                if (REF && !first && beta == 0.0)
-                {
-                    // the reference stops here (BaraffCloth.cpp:585-590)
-                    if (tid == 0)
-                        sh_st.final_check = 1;
-                    check = true;
-                    continue;
-                }
-                rho = rz;
-
-                // d = z + beta d_prev of the part's rows and of its halo
-                const T bt = (T)beta;
-                for (int i = 0; i < 3; i++)
-                {
-                    dv[i] = dir_value<T>(z[i], dv[i], bt, first);
-                    dl[3 * tid + i] = dv[i];
-                }
-                bool in_time = true;
-    #pragma clang loop unroll(disable)
-                for (int e = here(tid), n = 0; (e & ~63) < pt.halo_n && in_time; e += NT, n++)
-                {
-                    // (the first entries' z came with the sums)
-                    if (n > 0)
-                        in_time = await<3 * NP>(hz, z_tag, patience,
-                                                [&](int w) { return halo_word(words_z, e, w); });
-                    if (e < pt.halo_n)
-                    {
-                        T *p = dl + 3 * (NT + e);
-                        for (int i = 0; i < 3; i++)
-                            p[i] = dir_value<T>(Pieces<T>::join(hz + i * NP), p[i], bt, first);
-                    }
-                }
-                if (!in_time)
-                    sh_failed = 1;
-                if (!meet())
-                {
-                    failed = true;
-                    break;
-                }
-                // q = W d
-                T q[3];
-                ++tag;
-                if (MIXED && w64)
-                {
-                    // the FP64 matrix under FP32 vectors, from memory
-                    double y[3];
-                    product64(dl, y);
-                    for (int i = 0; i < 3; i++)
-                        q[i] = (T)y[i];
-                }
-                else
-                {
-                    T y[3][L] = {};
-                    auto slots = [&](auto first_slot, auto count) {
-                        constexpr int K0 = decltype(first_slot)::value, N = decltype(count)::value;
-                        T x[N][3];
-    #pragma unroll
-                        for (int k = 0; k < N; k++)
-                        {
-                            const unsigned at =
-                                (K0 + k) & 1 ? c[(K0 + k) / 2] >> 16 : c[(K0 + k) / 2] & 0xffff;
-                            const T *p = reinterpret_cast<const T *>(rs_lds + at);
-                            for (int i = 0; i < 3; i++)
-                                x[k][i] = p[i];
-                        }
-    #pragma unroll
-                        for (int k = 0; k < N; k++)
-                            for (int i = 0; i < 3; i++)
-                                y[i][(K0 + k) % L] +=
-                                    block<REF>(m[K0 + k][3 * i], m[K0 + k][3 * i + 1],
-                                               m[K0 + k][3 * i + 2], x[k][0], x[k][1], x[k][2]);
-                    };
-                    slots(std::integral_constant<int, 0>(), std::integral_constant<int, 9>());
-                    if (ws > 9)
-                        slots(std::integral_constant<int, 9>(),
-                              std::integral_constant<int, RS_SLOTS - 9>());
-                    // rows wider than the registers hold: the blocks in LDS, then
-                    // the rest from memory (a 20,011-point mesh with rows of up
-                    // to 21 blocks: 7.0 us an iteration, 8.5 with all of them
-                    // from memory)
-                    auto add = [&](int k, T (&t)[3]) __attribute__((always_inline)) {
-    #pragma unroll
-                        for (int j = 0; j < L; j++)
-                            if (k % L == j)
-                                for (int i = 0; i < 3; i++)
-                                    y[i][j] += t[i];
-                    };
-                    int k = RS_SLOTS;
-                    for (int kx = x0; kx < x0 + nx; kx++, k++)
-                    {
-                        const int me = here(lane);
-                        const T *x = reinterpret_cast<const T *>(rs_lds + cx[kx * SLICE + me]);
-                        const T *w = mx + 9 * kx * SLICE + me;
-                        T t[3];
-                        for (int i = 0; i < 3; i++)
-                            t[i] = block<REF>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
-                                              w[(3 * i + 2) * SLICE], x[0], x[1], x[2]);
-                        add(k, t);
-                    }
-    #pragma clang loop unroll(disable)
-                    for (; k < ws; k++)
-                    {
-                        const size_t at = (size_t)base + k * SLICE;
-                        const T *x = dl + 3 * (int)glob(rb.pos)[at + here(lane)];
-                        const G<T> *w = glob(Vecs<T>::W(d)) + 9 * at + here(lane);
-                        T t[3];
-                        for (int i = 0; i < 3; i++)
-                            t[i] = block<REF>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
-                                              w[(3 * i + 2) * SLICE], x[0], x[1], x[2]);
-                        add(k, t);
-                    }
-                    for (int i = 0; i < 3; i++)
-                        q[i] = phases<L>(y[i]);
-                }
-                publish(slice_sum<L>(block_row<double>((double)dv[0], (double)dv[1], (double)dv[2],
-                                                       (double)q[0], (double)q[1], (double)q[2])),
-                        64, 1, words_dq, sm_dq);
-                gather(1, words_dq, sm_dq, false);
-                if (!meet())
-                {
-                    failed = true;
-                    break;
-                }
-                double sq[1];
-                total(sm_dq, sq);
-                const double dq = sq[0];
-                if (REF ? dq == 0.0 || !isfinite(dq) : !(dq > 0.0) || !isfinite(dq))
-                {
-                    // d.Wd == 0 (BaraffCloth.cpp:547-551), or, to a tolerance, a
-                    // loss of definiteness: stop after a final true residual
-                    if (tid == 0)
-                    {
-                        sh_st.final_check = 1;
-                        sh_st.breakdown = dq == 0.0 ? 0 : 1;
-                    }
-                    check = due = true;
-                    continue;
-                }
-                // k_cg_update
-                const double alpha = uniform(rho / dq);
-                for (int i = 0; i < 3; i++)
-                {
-                    if constexpr (MIXED)
-                        x32[i] = x32[i] + (float)(alpha * (double)dv[i]);
-                    else
-                        x64[i] = fma_t(alpha, (double)dv[i], x64[i]);
-                    r[i] = (T)fma_t(-alpha, (double)q[i], (double)r[i]);
-                }
-                steps++;
+                // the reference stops here (BaraffCloth.cpp:585-590)
+                if (tid == 0)
+                    sh_st.final_check = 1;
+                check = true;
+                continue;
             }
-            again = false;
+            rho = rz;
+
+            // d = z + beta d_prev of the part's rows and of its halo
+            const T bt = (T)beta;
+            for (int i = 0; i < 3; i++)
+            {
+                dv[i] = dir_value<T>(z[i], dv[i], bt, first);
+                dl[3 * tid + i] = dv[i];
+            }
+            bool in_time = true;
+#pragma clang loop unroll(disable)
+            for (int e = here(tid), n = 0; (e & ~63) < pt.halo_n && in_time; e += NT, n++)
+            {
+                // (the first entries' z came with the sums)
+                if (n > 0)
+                    in_time = await<3 * NP>(hz, z_tag, patience,
+                                            [&](int w) { return halo_word(words_z, e, w); });
+                if (e < pt.halo_n)
+                {
+                    T *p = dl + 3 * (NT + e);
+                    for (int i = 0; i < 3; i++)
+                        p[i] = dir_value<T>(Pieces<T>::join(hz + i * NP), p[i], bt, first);
+                }
+            }
+            if (!in_time)
+                sh_failed = 1;
+            if (!meet())
+            {
+                failed = true;
+                break;
+            }
+            // q = W d
+            T q[3];
+            ++tag;
+            if (MIXED && w64)
+            {
+                // the FP64 matrix under FP32 vectors, from memory
+                double y[3];
+                product64(dl, y);
+                for (int i = 0; i < 3; i++)
+                    q[i] = (T)y[i];
+            }
+            else
+            {
+                T y[3][L] = {};
+                auto slots = [&](auto first_slot, auto count) {
+                    constexpr int K0 = decltype(first_slot)::value, N = decltype(count)::value;
+                    T x[N][3];
+#pragma unroll
+                    for (int k = 0; k < N; k++)
+                    {
+                        const unsigned at =
+                            (K0 + k) & 1 ? c[(K0 + k) / 2] >> 16 : c[(K0 + k) / 2] & 0xffff;
+                        const T *p = reinterpret_cast<const T *>(rs_lds + at);
+                        for (int i = 0; i < 3; i++)
+                            x[k][i] = p[i];
+                    }
+#pragma unroll
+                    for (int k = 0; k < N; k++)
+                        for (int i = 0; i < 3; i++)
+                            y[i][(K0 + k) % L] +=
+                                block<REF>(m[K0 + k][3 * i], m[K0 + k][3 * i + 1],
+                                           m[K0 + k][3 * i + 2], x[k][0], x[k][1], x[k][2]);
+                };
+                slots(std::integral_constant<int, 0>(), std::integral_constant<int, 9>());
+                if (ws > 9)
+                    slots(std::integral_constant<int, 9>(),
+                          std::integral_constant<int, RS_SLOTS - 9>());
+                // rows wider than the registers hold: the blocks in LDS, then
+                // the rest from memory (a 20,011-point mesh with rows of up
+                // to 21 blocks: 7.0 us an iteration, 8.5 with all of them
+                // from memory)
+                auto add = [&](int k, T (&t)[3]) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int j = 0; j < L; j++)
+                        if (k % L == j)
+                            for (int i = 0; i < 3; i++)
+                                y[i][j] += t[i];
+                };
+                int k = RS_SLOTS;
+                for (int kx = x0; kx < x0 + nx; kx++, k++)
+                {
+                    const int me = here(lane);
+                    const T *x = reinterpret_cast<const T *>(rs_lds + cx[kx * SLICE + me]);
+                    const T *w = mx + 9 * kx * SLICE + me;
+                    T t[3];
+                    for (int i = 0; i < 3; i++)
+                        t[i] = block<REF>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
+                                          w[(3 * i + 2) * SLICE], x[0], x[1], x[2]);
+                    add(k, t);
+                }
+#pragma clang loop unroll(disable)
+                for (; k < ws; k++)
+                {
+                    const size_t at = (size_t)base + k * SLICE;
+                    const T *x = dl + 3 * (int)glob(rb.pos)[at + here(lane)];
+                    const G<T> *w = glob(Vecs<T>::W(d)) + 9 * at + here(lane);
+                    T t[3];
+                    for (int i = 0; i < 3; i++)
+                        t[i] = block<REF>(w[(3 * i) * SLICE], w[(3 * i + 1) * SLICE],
+                                          w[(3 * i + 2) * SLICE], x[0], x[1], x[2]);
+                    add(k, t);
+                }
+                for (int i = 0; i < 3; i++)
+                    q[i] = phases<L>(y[i]);
+            }
+            publish(slice_sum<L>(block_row<double>((double)dv[0], (double)dv[1], (double)dv[2],
+                                                   (double)q[0], (double)q[1], (double)q[2])),
+                    64, 1, words_dq, sm_dq);
+            gather(1, words_dq, sm_dq, false);
+            if (!meet())
+            {
+                failed = true;
+                break;
+            }
+            double sq[1];
+            total(sm_dq, sq);
+            const double dq = sq[0];
+            if (REF ? dq == 0.0 || !isfinite(dq) : !(dq > 0.0) || !isfinite(dq))
+            {
+                // d.Wd == 0 (BaraffCloth.cpp:547-551), or, to a tolerance, a
+                // loss of definiteness: stop after a final true residual
+                if (tid == 0)
+                {
+                    sh_st.final_check = 1;
+                    sh_st.breakdown = dq == 0.0 ? 0 : 1;
+                }
+                check = due = true;
+                continue;
+            }
+            // k_cg_update
+            const double alpha = uniform(rho / dq);
             double v[2] = {0.0, 0.0};
             for (int i = 0; i < 3; i++)
             {
+                if constexpr (MIXED)
+                    x32[i] = x32[i] + (float)(alpha * (double)dv[i]);
+                else
+                    x64[i] = fma_t(alpha, (double)dv[i], x64[i]);
+                r[i] = (T)fma_t(-alpha, (double)q[i], (double)r[i]);
                 z[i] = P[i] * r[i];
                 v[0] = fma_t((double)r[i], (double)z[i], v[0]);
                 v[1] = fma_t((double)r[i], (double)r[i], v[1]);
@@ -951,6 +956,7 @@ k_resident(ResidentLaunch a)
             total(sm_rz, t);
             rz = t[0];
             rr = t[1];
+            steps++;
             first = false;
             if constexpr (!MIXED)
                 if (steps % PROGRESS == 0 && pt.slice0 == pt.set0 && tid == 0)
@@ -993,7 +999,11 @@ k_resident(ResidentLaunch a)
             st.rho = rho;
             st.first = first;
             if (PAUSE && paused)
+            {
                 st.since = steps;
+                st.rr = rr;
+                st.rr_true = rz;
+            }
             st.iter = st.total;
             store_state(glob(d.cg) + 2 * inst, st);
             store_state(glob(d.cg) + 2 * inst + 1, st);
