@@ -1234,8 +1234,9 @@ int Batch::upload_lists(Lane &L)
 // the others while all of them solve; in lanes of their own they run at the
 // pace of their own launches, alongside the others' bandwidth-bound ones,
 // and a step ends when its slowest lane does.  Each cloth's arithmetic is
-// its own, so results are bit-identical to one chain.  One chain when
-// BW_LANES=0, on the first solve, for fewer than 8 cloths, with group sums
+// its own, so results are bit-identical to one chain.  The cloths are those
+// that one launch has not solved (resident.hip).  One chain when BW_LANES=0, on
+// the first solve, for fewer than 8 such cloths, with group sums
 // (whose launch covers every cloth's groups) and in bw_batch_step_noalloc
 // (lanes 1 and 2 allocate streams and buffers on first use).  Returns the
 // number of lanes.
@@ -1243,21 +1244,23 @@ int Batch::plan_lanes()
 {
     const char *env = std::getenv("BW_LANES");
     const bool lanes_rule = env ? std::atoi(env) != 0 : true;
-    const int n = size();
     lanes_[0].members.clear();
-    const int left = (int)std::count(solved_.begin(), solved_.end(), 0);
-    if (!lanes_rule || !lanes_allowed_ || left < 8 || left < n || d_.n_groups > 0 ||
-        (int)pred_launches_.size() != n)
+    // the cloths that this step's one launch has not solved
+    std::vector<int> &order = lane_order_;
+    order.clear();
+    bool known = (int)pred_launches_.size() == size();
+    for (int i = 0; i < size(); i++)
+        if (!solved_[i])
+        {
+            order.push_back(i);
+            known = known && pred_launches_[i] > 0;
+        }
+    const int n = (int)order.size();
+    if (!lanes_rule || !lanes_allowed_ || n < 8 || d_.n_groups > 0 || !known)
     {
-        for (int i = 0; i < n; i++)
-            if (!solved_[i])
-                lanes_[0].members.push_back(i);
+        lanes_[0].members = order;
         return 1;
     }
-    std::vector<int> &order = lane_order_;
-    order.resize(n);
-    for (int i = 0; i < n; i++)
-        order[i] = i;
     std::stable_sort(order.begin(), order.end(),
                      [&](int a, int b) { return pred_launches_[a] > pred_launches_[b]; });
     int a = std::max(1, n / 10), b = std::max(1, n / 3);

@@ -43,7 +43,7 @@ def _run(monkeypatch, cloths, steps, resident, **env):
     return out, st
 
 
-ONE_LAUNCH, LAUNCHES = 2, 0  # solve_route
+ONE_LAUNCH, LANES, LAUNCHES = 2, 1, 0  # solve_route
 
 
 def _same(a, b, route=ONE_LAUNCH):
@@ -197,6 +197,20 @@ def test_given_up_launch_keeps_the_rounding(monkeypatch, env):
         assert a[1][0]["matrix_fp64"] == b[1][0]["matrix_fp64"] == bool(env)
         assert a[1][0]["solve_route"] == LAUNCHES and b[1][0]["solve_route"] == ONE_LAUNCH
         assert np.array_equal(a[0][0], b[0][0])
+
+
+def test_lanes_beside_one_launch(monkeypatch):
+    """8 clothes whose parts' halos are too long for one launch (their rows
+    sorted over the whole mesh) solve in lanes, and the ninth in one launch"""
+    monkeypatch.setenv("BW_SORT_WINDOW", "65536")
+    monkeypatch.setenv("BW_SPMV_LPR", "1")
+    cloths = [_delaunay(7000 + 100 * k, "mixed") for k in range(8)] + [_grid(9, 9, "mixed")]
+    a = _run(monkeypatch, cloths, 2, "1")
+    b = _run(monkeypatch, cloths, 2, "1", BW_LANES="0")
+    assert [s["solve_route"] for s in a[1]] == 8 * [LANES] + [ONE_LAUNCH]
+    assert [s["solve_route"] for s in b[1]] == 8 * [LAUNCHES] + [ONE_LAUNCH]
+    for x, y in zip(a[0], b[0]):
+        assert np.array_equal(x, y)
 
 
 # the last three: clothes of 11, 17 and 66 parts, from where the parts' sums of
