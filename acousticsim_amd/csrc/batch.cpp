@@ -34,12 +34,12 @@ void check(hipError_t e, const char *what)
 // group sums and 21.0 with).  The server's cloths share their rounds'
 // launches, where group sums pay off from 512 slices (a serving mix ran 42.6
 // cloth-steps/s at 512 against 32.0 at 2048); those that one launch solves
-// (resident.hip) have no use for them.
-static int group_min(bool shared_launches)
+// (resident.hip: up to 1,088 slices) have no use for them.
+static int group_min(bool shared_launches, bool one_launch)
 {
     if (const char *e = std::getenv("BW_GROUP_MIN"))
         return std::max(0, std::atoi(e));
-    return shared_launches ? RS_SETS_CAP : 2048;
+    return shared_launches && !one_launch ? 512 : 2048;
 }
 
 void *Batch::dalloc_raw(size_t bytes)
@@ -317,9 +317,6 @@ void Batch::build_layout()
     std::vector<double> ie_factor(nie);
     std::vector<InstParams> params(n);
     std::vector<int> group_inst;
-    // a batch's own rule does not depend on its other members, so that a
-    // cloth gives the same result alone and in a mix
-    const int gmin = group_min(opt_.shared_launches);
     for (int i = 0; i < n; i++)
     {
         const ClothModel &m = models_[i];
@@ -438,6 +435,14 @@ void Batch::build_layout()
         P.blk_count = nslices_[i] / BW_SB;
         P.slice_begin = slice_base_[i];
         P.slice_count = nslices_[i];
+    }
+    const ResidentLists resident = plan_resident(col, slice_off, slice_w, params);
+    for (int i = 0; i < n; i++)
+    {
+        InstParams &P = params[i];
+        // a batch's own rule does not depend on its other members, so that a
+        // cloth gives the same result alone and in a mix
+        const int gmin = group_min(opt_.shared_launches, resident_.count[i] > 0);
         // group sums for cloths whose per-workgroup pass over all slice
         // partials would cost more than one extra small launch
         P.group_begin = (int)group_inst.size();
@@ -692,8 +697,7 @@ void Batch::build_layout()
     upload(d_.ie_rows, ie_rows);
     upload(d_.ie_factor, ie_factor);
     upload(d_.params, params);
-    if (kind_ != SolverKind::GpuForm)
-        build_resident(col, slice_off, slice_w, params);
+    build_resident(resident);
     // initial state: rest positions, at rest
     for (int i = 0; i < n; i++)
     {

@@ -247,12 +247,20 @@ private:
     void solve_ref(const std::function<void()> &again);
     void solve_cg(const std::function<void()> &again);
     void take_stats(int i, const CgState &s, SolveRoute route);
-    // One-launch solves (resident_plan.cpp).  build_resident: the cloths
-    // that fit them as parts, given the layout's columns; solve_resident:
-    // one launch over those cloths, false when it was given up and all
-    // states are again those of a solve's start
-    void build_resident(const std::vector<int> &col, const std::vector<int> &slice_off,
-                        const std::vector<int> &slice_w, const std::vector<InstParams> &params);
+    // One-launch solves (resident_plan.cpp).  plan_resident: the cloths that
+    // fit them as parts, given the layout's columns; build_resident: their
+    // device arrays; solve_resident: one launch over those cloths, false when
+    // it was given up and all states are again those of a solve's start
+    struct ResidentLists
+    {
+        std::vector<ResidentPart> part;
+        std::vector<int> halo_row;
+        std::vector<uint16_t> pos;
+    };
+    ResidentLists plan_resident(const std::vector<int> &col, const std::vector<int> &slice_off,
+                                const std::vector<int> &slice_w,
+                                const std::vector<InstParams> &params);
+    void build_resident(const ResidentLists &lists);
     bool solve_resident(const std::function<void()> &again);
     bool all_resident() const;
     void free_resident();

@@ -88,10 +88,13 @@ void resident_limits(ResidentLaunch &a, ResidentCtl &ctl)
 }
 
 // Parts of each cloth that fits: its slices in order, as many to a
-// workgroup as it holds.  BW_RESIDENT=0 turns one-launch solves off.
-void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &slice_off,
-                           const std::vector<int> &slice_w,
-                           const std::vector<InstParams> &params)
+// workgroup as it holds.  BW_RESIDENT=0 turns one-launch solves off;
+// BW_GROUP_MIN leaves the cloths above it to the launches, whose order of sums
+// it fixes.
+Batch::ResidentLists Batch::plan_resident(const std::vector<int> &col,
+                                          const std::vector<int> &slice_off,
+                                          const std::vector<int> &slice_w,
+                                          const std::vector<InstParams> &params)
 {
     const bool fp32 = kind_ == SolverKind::CG32;
     const int hold = resident_slices(fp32);
@@ -99,12 +102,15 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
     rp = ResidentPlan();
     rp.first.assign(size(), 0);
     rp.count.assign(size(), 0);
+    ResidentLists lists;
+    std::vector<ResidentPart> &part = lists.part;
+    std::vector<int> &halo_row = lists.halo_row, rows;
+    std::vector<uint16_t> &pos = lists.pos;
     // (words are addressed by 32-bit byte offsets)
-    if (d_.n_rows > (1 << 26) || env_int("BW_RESIDENT", 1) == 0)
-        return;
-    std::vector<ResidentPart> part;
-    std::vector<int> halo_row, rows;
-    std::vector<uint16_t> pos(col.size(), 0);
+    if (kind_ == SolverKind::GpuForm || d_.n_rows > (1 << 26) || env_int("BW_RESIDENT", 1) == 0)
+        return lists;
+    const int slices_cap = std::min(RS_SETS_CAP, env_int("BW_GROUP_MIN", RS_SETS_CAP));
+    pos.assign(col.size(), 0);
     // per row: the last part that met it, and its place among that part's
     // directions (own rows, then the halo)
     std::vector<int> met(d_.n_rows, -1);
@@ -113,7 +119,7 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
     for (int i = 0; i < size(); i++)
     {
         const int n = nslices_[i], count = (n + hold - 1) / hold;
-        if (n > RS_SETS_CAP || count > PARTS_CAP || params[i].group_count > 0 || params[i].max_iter > ITER_CAP)
+        if (n > slices_cap || count > PARTS_CAP || params[i].max_iter > ITER_CAP)
             continue;
         const size_t part0 = part.size(), halo0 = halo_row.size();
         int longest = 0, s = slice_base_[i];
@@ -179,6 +185,13 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
         }
     }
     rp.parts = (int)part.size();
+    return lists;
+}
+
+void Batch::build_resident(const ResidentLists &lists)
+{
+    const bool fp32 = kind_ == SolverKind::CG32;
+    ResidentPlan &rp = resident_;
     if (rp.parts == 0)
         return;
     auto put = [](auto *dst, const auto &v) {
@@ -187,12 +200,12 @@ void Batch::build_resident(const std::vector<int> &col, const std::vector<int> &
                   "hipMemcpy H2D");
     };
     typedef unsigned long long u64;
-    auto *d_part = dalloc<ResidentPart>(part.size());
-    auto *d_halo = dalloc<int>(halo_row.size());
-    auto *d_pos = dalloc<uint16_t>(pos.size());
-    put(d_part, part);
-    put(d_halo, halo_row);
-    put(d_pos, pos);
+    auto *d_part = dalloc<ResidentPart>(lists.part.size());
+    auto *d_halo = dalloc<int>(lists.halo_row.size());
+    auto *d_pos = dalloc<uint16_t>(lists.pos.size());
+    put(d_part, lists.part);
+    put(d_halo, lists.halo_row);
+    put(d_pos, lists.pos);
     ResidentBatch rb;
     rb.d = d_;
     rb.part = d_part;

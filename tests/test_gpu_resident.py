@@ -285,6 +285,24 @@ def test_served_same_bits(monkeypatch, precision, pause, env):
         s.close()
 
 
+def test_served_by_launches_takes_group_sums(monkeypatch):
+    """a served cloth of 520 slices that goes by launches has the sums of those
+    above 512 slices, in groups of slices: the bits of a batch with group sums,
+    not of one without (in FP64: float vectors round the difference away)"""
+    cloth = _grid(182, 182, "fp64", 0.1)
+    monkeypatch.setenv("BW_RESIDENT", "0")
+    monkeypatch.setenv("BW_SPMV_LPR", "1")
+    s = capi.Server(budget_bytes=4e9, max_resident=2, precision="fp64")
+    rid = s.submit(cloth[0], cloth[1], 2)
+    assert s.wait(rid, 60.0) and s.info(rid)["status"] == 0
+    x = s.get_pos(rid)
+    s.close()
+    monkeypatch.setenv("BW_STAGE_LDS", "p99")
+    same = [np.array_equal(x, _run(monkeypatch, [cloth], 2, "0", BW_GROUP_MIN=g)[0][0])
+            for g in ("512", "2048")]
+    assert same == [True, False]
+
+
 @pytest.mark.parametrize("precision", ["mixed", "fp64"])
 def test_served_short_solves_do_not_wait_for_long_ones(precision):
     """20 steps of a 9 x 9 cloth beside a stiff 129 x 129 one whose step takes
