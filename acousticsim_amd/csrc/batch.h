@@ -70,6 +70,8 @@ struct BatchOptions
     // the batch's solver launches are shared with other batches (a server's
     // rounds): group sums pay off from smaller cloths
     bool shared_launches = false;
+    // one-launch solves where they fit (their arrays take some 5% more memory)
+    bool one_launch = true;
 };
 
 class Batch

@@ -107,7 +107,8 @@ Batch::ResidentLists Batch::plan_resident(const std::vector<int> &col,
     std::vector<int> &halo_row = lists.halo_row, rows;
     std::vector<uint16_t> &pos = lists.pos;
     // (words are addressed by 32-bit byte offsets)
-    if (kind_ == SolverKind::GpuForm || d_.n_rows > (1 << 26) || env_int("BW_RESIDENT", 1) == 0)
+    if (!opt_.one_launch || kind_ == SolverKind::GpuForm || d_.n_rows > (1 << 26) ||
+        env_int("BW_RESIDENT", 1) == 0)
         return lists;
     const int slices_cap = std::min(RS_SETS_CAP, env_int("BW_GROUP_MIN", RS_SETS_CAP));
     pos.assign(col.size(), 0);

@@ -20,8 +20,9 @@ void check(hipError_t e, const char *what)
 }
 
 // Device bytes a one-cloth Batch will allocate, from the model alone (an
-// upper bound: the ELL slots are counted at the widest row).
-size_t estimate_bytes(const ClothModel &m)
+// upper bound: the ELL slots are counted at the widest row), with the arrays
+// of one-launch solves or without.
+size_t estimate_bytes(const ClothModel &m, bool one_launch)
 {
     int wmax = 0;
     for (int v = 0; v < m.nv; v++)
@@ -40,7 +41,7 @@ size_t estimate_bytes(const ClothModel &m)
     b += (size_t)m.nv * 4 * 4 + (size_t)m.nnzb() * 4 * 3;
     b += ((size_t)9 * m.nt + 16 * nie) * 4 + ((size_t)3 * m.nt + 4 * nie) * 4 * 2;
     b += (size_t)m.nt * (3 * 4 + 4 + 12 * 4 + 4 + 25 * 8) + nie * (4 * 4 + 8 + 25 * 8);
-    if (slices <= (size_t)RS_SETS_CAP) // one-launch solves: positions, exchange words, halos
+    if (one_launch && slices <= (size_t)RS_SETS_CAP) // positions, exchange words, halos
         b += entries * 2 + rows * (6 + 6) * 8 + slices * 12 * 8 +
              slices * (sizeof(ResidentPart) + 4 * (size_t)RS_HALO32 / RS_WAVES64);
     return b + (1 << 20);
@@ -215,7 +216,14 @@ void Server::builder_loop()
                                          (opt_.fp32 ? "mixed" : "fp64") + "\" requests");
             if (!job.x0.empty() && job.x0.size() != 3 * (size_t)m.nv)
                 throw std::runtime_error("config: x0 must hold 3 doubles per vertex");
-            const size_t est = estimate_bytes(m);
+            // (a request that fits the budget by launches only is solved so)
+            bool one_launch = true;
+            size_t est = estimate_bytes(m, true);
+            if (est > opt_.budget_bytes)
+            {
+                one_launch = false;
+                est = estimate_bytes(m, false);
+            }
             if (est > opt_.budget_bytes)
                 throw std::runtime_error("capacity: request needs more device memory than the budget");
             {
@@ -235,6 +243,7 @@ void Server::builder_loop()
             bo.stream = stream_;
             bo.cg_states = states_dev_ + 2 * (size_t)slot;
             bo.shared_launches = true;
+            bo.one_launch = one_launch;
             std::vector<ClothModel> ms;
             ms.push_back(std::move(m));
             auto r = std::make_unique<Resident>();

@@ -303,6 +303,29 @@ def test_served_by_launches_takes_group_sums(monkeypatch):
     assert same == [True, False]
 
 
+def test_served_within_a_budget_without_room_for_one_launch(monkeypatch):
+    """a budget that holds a request, but not the arrays of its one-launch
+    solves, serves it by launches, with the same bits"""
+    cloth = _grid(33, 33, "mixed")
+    monkeypatch.setenv("BW_SPMV_LPR", "1")
+
+    def serve(budget):
+        s = capi.Server(budget_bytes=budget, max_resident=2, precision="mixed")
+        rid = s.submit(cloth[0], cloth[1], 2)
+        s.wait(rid, 60.0)
+        info = s.info(rid)
+        x = s.get_pos(rid) if info["status"] == 0 else None
+        launches = s.counters()["launches"]
+        s.close()
+        return info, x, launches
+    full, x, few = serve(1e9)
+    tight, y, many = serve(full["admitted_bytes"] - 1)
+    assert full["status"] == tight["status"] == 0 and np.array_equal(x, y)
+    assert few < 100 < tight["pcg_iterations"] < many
+    assert tight["device_bytes"] <= tight["admitted_bytes"] < full["admitted_bytes"]
+    assert serve(tight["admitted_bytes"] - 1)[0]["status"] == -5  # BW_ERR_CAPACITY
+
+
 @pytest.mark.parametrize("precision", ["mixed", "fp64"])
 def test_served_short_solves_do_not_wait_for_long_ones(precision):
     """20 steps of a 9 x 9 cloth beside a stiff 129 x 129 one whose step takes
