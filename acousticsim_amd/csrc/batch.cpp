@@ -169,12 +169,14 @@ Batch::Batch(std::vector<ClothModel> models, const BatchOptions &opt)
     if (const char *g = std::getenv("BW_GRAPHS"))
         graphs_disabled_ = std::string(g) == "0";
     use_graphs_ = !graphs_disabled_;
-    check(hipHostMalloc((void **)&host_state_, sizeof(InstState) * models_.size()),
-          "hipHostMalloc");
+    if (kind_ == SolverKind::RefPCG64)
+        check(hipHostMalloc((void **)&host_state_, sizeof(InstState) * models_.size()),
+              "hipHostMalloc");
     check(hipHostMalloc((void **)&host_cg_, 2 * sizeof(CgState) * models_.size()),
           "hipHostMalloc");
-    check(hipHostMalloc((void **)&host_gf_, 2 * sizeof(GfState) * models_.size()),
-          "hipHostMalloc");
+    if (kind_ == SolverKind::GpuForm)
+        check(hipHostMalloc((void **)&host_gf_, 2 * sizeof(GfState) * models_.size()),
+              "hipHostMalloc");
     if (kind_ == SolverKind::GpuForm)
         tuned_ = true; // one SpMV form
     build_layout();
@@ -487,18 +489,27 @@ void Batch::build_layout()
     std::vector<uint16_t> lcol(entries);
     {
         int hmax = 0;
-        std::vector<int> u;
+        // per row: the last slice that met it, and its place in that slice's list
+        std::vector<int> u, met(d_.n_rows, -1);
+        std::vector<uint16_t> place(d_.n_rows, 0);
         for (int s = 0; s < slices; s++)
         {
             const size_t e0 = slice_off[s], e1 = e0 + (size_t)slice_w[s] * SLICE;
-            u.assign(col.begin() + e0, col.begin() + e1);
+            u.clear();
+            for (size_t e = e0; e < e1; e++)
+                if (met[col[e]] != s)
+                {
+                    met[col[e]] = s;
+                    u.push_back(col[e]);
+                }
             std::sort(u.begin(), u.end());
-            u.erase(std::unique(u.begin(), u.end()), u.end());
             hmax = std::max(hmax, (int)u.size());
             if (hmax > HALO_CAP)
                 break;
+            for (size_t k = 0; k < u.size(); k++)
+                place[u[k]] = (uint16_t)k;
             for (size_t e = e0; e < e1; e++)
-                lcol[e] = (uint16_t)(std::lower_bound(u.begin(), u.end(), col[e]) - u.begin());
+                lcol[e] = place[col[e]];
             halo_row.insert(halo_row.end(), u.begin(), u.end());
             halo_off[s + 1] = (int)halo_row.size();
         }

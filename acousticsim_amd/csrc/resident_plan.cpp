@@ -195,37 +195,53 @@ void Batch::build_resident(const ResidentLists &lists)
     ResidentPlan &rp = resident_;
     if (rp.parts == 0)
         return;
-    auto put = [](auto *dst, const auto &v) {
-        if (!v.empty())
-            check(hipMemcpy(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice),
-                  "hipMemcpy H2D");
-    };
+    // one allocation for all arrays (each costs a fill and a wait), the ones
+    // with contents first, uploaded together
     typedef unsigned long long u64;
-    auto *d_part = dalloc<ResidentPart>(lists.part.size());
-    auto *d_halo = dalloc<int>(lists.halo_row.size());
-    auto *d_pos = dalloc<uint16_t>(lists.pos.size());
-    put(d_part, lists.part);
-    put(d_halo, lists.halo_row);
-    put(d_pos, lists.pos);
-    ResidentBatch rb;
+    size_t bytes = 0;
+    auto place = [&](size_t n) {
+        const size_t at = bytes;
+        bytes += (n + 255) & ~(size_t)255;
+        return at;
+    };
+    auto size_of = [](const auto &v) { return v.size() * sizeof(v[0]); };
+    const size_t rows = d_.n_rows, slices = d_.n_slices;
+    const size_t part = place(size_of(lists.part)), halo = place(size_of(lists.halo_row)),
+                 pos = place(size_of(lists.pos)), table = place(sizeof(ResidentBatch)),
+                 contents = bytes;
+    const size_t z = place(rows * 3 * (fp32 ? 1 : 2) * sizeof(u64)),
+                 x = place(rows * 6 * sizeof(u64)), s_dq = place(slices * 2 * sizeof(u64)),
+                 s_rz = place(slices * 4 * sizeof(u64)), s_res = place(slices * 6 * sizeof(u64)),
+                 epoch = place(size() * sizeof(unsigned));
+    const size_t ctl_bytes = sizeof(ResidentCtl) + (size_t)rp.parts * sizeof(int2);
+    const size_t ctl = place(ctl_bytes);
+    char *base = dalloc<char>(bytes);
+    ResidentBatch &rb = rp.entry;
     rb.d = d_;
-    rb.part = d_part;
-    rb.halo_row = d_halo;
-    rb.pos = d_pos;
-    rb.z = dalloc<u64>((size_t)d_.n_rows * 3 * (fp32 ? 1 : 2));
-    rb.x = dalloc<u64>((size_t)d_.n_rows * 6);
-    rb.s_dq = dalloc<u64>((size_t)d_.n_slices * 2);
-    rb.s_rz = dalloc<u64>((size_t)d_.n_slices * 4);
-    rb.s_res = dalloc<u64>((size_t)d_.n_slices * 6);
-    rb.epoch = dalloc<unsigned>(size());
-    rp.entry = rb;
+    rb.part = reinterpret_cast<ResidentPart *>(base + part);
+    rb.halo_row = reinterpret_cast<int *>(base + halo);
+    rb.pos = reinterpret_cast<uint16_t *>(base + pos);
+    rb.z = reinterpret_cast<u64 *>(base + z);
+    rb.x = reinterpret_cast<u64 *>(base + x);
+    rb.s_dq = reinterpret_cast<u64 *>(base + s_dq);
+    rb.s_rz = reinterpret_cast<u64 *>(base + s_rz);
+    rb.s_res = reinterpret_cast<u64 *>(base + s_res);
+    rb.epoch = reinterpret_cast<unsigned *>(base + epoch);
+    std::vector<char> head(contents);
+    auto put = [&](size_t at, const void *src, size_t n) {
+        if (n)
+            std::memcpy(head.data() + at, src, n);
+    };
+    put(part, lists.part.data(), size_of(lists.part));
+    put(halo, lists.halo_row.data(), size_of(lists.halo_row));
+    put(pos, lists.pos.data(), size_of(lists.pos));
+    put(table, &rb, sizeof rb);
+    check(hipMemcpy(base, head.data(), contents, hipMemcpyHostToDevice), "hipMemcpy H2D");
     if (opt_.shared_launches)
         return; // the server has the table and the tickets
-    rp.table = dalloc<ResidentBatch>(1);
-    check(hipMemcpy(rp.table, &rb, sizeof rb, hipMemcpyHostToDevice), "hipMemcpy H2D");
-    const size_t ctl = sizeof(ResidentCtl) + (size_t)rp.parts * sizeof(int2);
-    rp.ctl = dalloc<char>(ctl);
-    check(hipHostMalloc((void **)&rp.host_ctl, ctl), "hipHostMalloc");
+    rp.table = reinterpret_cast<ResidentBatch *>(base + table);
+    rp.ctl = base + ctl;
+    check(hipHostMalloc((void **)&rp.host_ctl, ctl_bytes), "hipHostMalloc");
 }
 
 void Batch::free_resident()
