@@ -431,6 +431,7 @@ void Batch::build_layout()
         P.carry = 1;
         if (const char *e = std::getenv("BW_STALL_CARRY"))
             P.carry = std::max(1, std::atoi(e));
+        carry_ = P.carry;
         P.gf_a = m.cfg.rayleigh_a;
         P.gf_b = m.cfg.rayleigh_b;
         P.blk_begin = slice_base_[i] / BW_SB;
@@ -677,6 +678,7 @@ void Batch::build_layout()
     sched_pairs_.reserve(models_.size());
     lane_order_.reserve(models_.size());
     solved_.reserve(models_.size());
+    w64_next_.assign(models_.size(), 0);
     pred_launches_.reserve(models_.size());
     drag_vertex_.assign(models_.size(), -1);
     ydrag_.assign(models_.size(), 0.0f);
@@ -734,6 +736,10 @@ void Batch::mark_fresh(int i)
 {
     if (!d_.cg_fresh)
         return;
+    if (i >= 0)
+        w64_next_[i] = 0;
+    else
+        std::fill(w64_next_.begin(), w64_next_.end(), 0);
     const unsigned char one[1] = {1};
     if (i >= 0)
         check(hipMemcpy(d_.cg_fresh + i, one, 1, hipMemcpyHostToDevice), "hipMemcpy fresh");
@@ -1385,6 +1391,7 @@ void Batch::take_stats(int i, const CgState &s, SolveRoute route)
     st.pcg_iterations = s.total;
     st.outer_iterations = s.updates;
     st.matrix_fp64 = s.w64;
+    w64_next_[i] = s.w64 && s.stalls + 1 >= carry_; // (k_cg_reset)
     st.rel_residual = s.bb > 0 ? std::sqrt(s.rr_true / s.bb) : std::sqrt(s.rr_true);
     // launches this cloth needed: two per iteration and per true residual
     pred_launches_[i] = 2LL * (s.total + s.updates) + 2;
@@ -1395,7 +1402,8 @@ void Batch::solve_cg(const std::function<void()> &again)
     launch_cg_reset(d_, stream_);
     // the cloths that one launch solves; the launches below take the others
     solved_.assign(size(), 0);
-    if (resident_.parts > 0 && lanes_allowed_ && !resident_.given_up && solve_resident(again))
+    if (resident_.parts > 0 && lanes_allowed_ && !resident_.given_up && !w64_by_launches() &&
+        solve_resident(again))
     {
         read_states(lanes_[0]);
         bool all = true;

@@ -227,6 +227,8 @@ private:
     hipEvent_t lanes_start_ = nullptr;
     bool lanes_allowed_ = true; // false inside bw_batch_step_noalloc
     std::vector<int> lane_order_;
+    int carry_ = 1;            // InstParams::carry
+    std::vector<char> w64_next_; // per cloth: its next solve starts on the FP64 matrix
     std::vector<char> solved_; // per cloth: this solve's one launch has solved it
     int plan_lanes();
     void open_lane(Lane &L);
@@ -265,6 +267,7 @@ private:
     void build_resident(const ResidentLists &lists);
     bool solve_resident(const std::function<void()> &again);
     bool all_resident() const;
+    bool w64_by_launches() const;
     void free_resident();
     struct ResidentPlan
     {

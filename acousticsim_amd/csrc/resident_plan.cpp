@@ -261,6 +261,25 @@ bool Batch::all_resident() const
     return true;
 }
 
+// Solves that start on the FP64 matrix (after a stall in the step before) go by
+// launches where those are faster: the one launch reads that matrix with a CU a
+// part only.  us an iteration, one launch and launches (1 lane per row): 33 x 33
+// 11.5 and 9.1, 65 x 65 11.9 and 10.0, 125 x 125 12.1 and 10.1, 210 x 210 (692
+// slices) 17.4 and 16.3, 257 x 257 18.5 and 19.6, one part (21 x 21) 8.2 and 9.5;
+// 2 of 97 x 97 (296 slices) 12.1 and 11.2, 5 of 65 x 65 (340) 11.6 and 11.2, 2 of
+// 125 x 125 (496) 12.3 and 12.6; 8 of 33 x 33 11.3 and 11.9.  A batch whose other
+// cloths go in the one launch keeps these there, beside them.
+bool Batch::w64_by_launches() const
+{
+    if (kind_ != SolverKind::CG32 || size() >= 8 || resident_.most <= 1 ||
+        d_.n_slices > (size() == 1 ? 700 : 350))
+        return false;
+    for (char w : w64_next_)
+        if (!w)
+            return false;
+    return true;
+}
+
 // One launch over the resident cloths, after the reset of their states on
 // the batch's stream.  Cloths go in the order of the iterations that they
 // took in the last solve, the most first (in the first solve: of their

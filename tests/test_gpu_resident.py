@@ -114,7 +114,41 @@ def test_fp64_matrix_same_bits(monkeypatch):
     env = dict(BW_MAX_SINCE="20", BW_STALL="1e-9")
     a, b = (_run(monkeypatch, cloths, 2, r, **env) for r in "10")
     assert all(s["matrix_fp64"] for s in a[1])
-    _same(a, b)
+    _same(a, b, LAUNCHES)  # the second step; the first is in one launch
+
+
+# one part; several; more slices than launches are faster for; 8 cloths; some
+# cloths on the FP32 matrix, so that the others stay beside them
+@pytest.mark.parametrize("sides,route", [((21,), ONE_LAUNCH), ((30,), LAUNCHES), ((65, 30), LAUNCHES),
+                                         ((97, 97, 97), ONE_LAUNCH), (8 * (30,), ONE_LAUNCH),
+                                         ((65, 5), ONE_LAUNCH)])
+def test_fp64_matrix_route(monkeypatch, sides, route):
+    """steps that start on the FP64 matrix, by the route that is faster there,
+    and back after the state is set, with the same bits"""
+    cloths = [_grid(n, n, "mixed") for n in sides]
+    monkeypatch.setenv("BW_SPMV_LPR", "1")
+    # (a 5 x 5 cloth's checks all come within this window)
+    monkeypatch.setenv("BW_MAX_SINCE", "20")
+    monkeypatch.setenv("BW_STALL", "1e-9")
+    out = []
+    for resident in "10":
+        monkeypatch.setenv("BW_RESIDENT", resident)
+        b = capi.ClothBatch([c for c, _ in cloths], [x for _, x in cloths])
+        b.step(3)
+        st = [b.stats(i) for i in range(b.n)]
+        assert [s["matrix_fp64"] for s in st] == [int(n > 5) for n in sides]
+        x = [b.get_pos(i) for i in range(b.n)]
+        for i in range(b.n):
+            b.set_state(i, x[i], x[i])
+        b.step(1)
+        out.append(([s["solve_route"] for s in st], [b.stats(i)["solve_route"] for i in range(b.n)],
+                    x, [b.get_pos(i) for i in range(b.n)]))
+        b.close()
+    assert out[0][0] == len(sides) * [route] and out[0][1] == len(sides) * [ONE_LAUNCH]
+    assert not any(r == ONE_LAUNCH for r in out[1][0] + out[1][1])
+    for k in (2, 3):
+        for p, q in zip(out[0][k], out[1][k]):
+            assert np.array_equal(p, q)
 
 
 def test_more_parts_than_the_chip_holds(monkeypatch):
@@ -188,9 +222,11 @@ def test_given_up_launch_solves_by_launches(monkeypatch):
 def test_given_up_launch_keeps_the_rounding(monkeypatch, env):
     """the steps after a launch that gave up, whose launches are then tuned,
     are those of one-launch solves (no variant fixed by the environment: the
-    tuner alone picks 4 lanes for the first cloth and 2 for the second), also
-    of a cloth that stays on the FP64 matrix from step to step"""
-    cloths = [_grid(30, 31, "mixed"), _grid(45, 45, "mixed", 5.0)]
+    tuner alone picks 4 lanes for the first two clothes and 2 for the third),
+    also of a cloth that stays on the FP64 matrix from step to step"""
+    cloths = [_grid(21, 21, "mixed")]
+    if not env:
+        cloths += [_grid(30, 31, "mixed"), _grid(45, 45, "mixed", 5.0)]
     for cloth in cloths:
         a = _run(monkeypatch, [cloth], 3, "1", BW_RESIDENT_GIVE_UP="150", **env)
         b = _run(monkeypatch, [cloth], 3, "1", **env)
