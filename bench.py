@@ -13,10 +13,12 @@ Reported beside it, in the same run:
   * step latency p50 / p99 (per batch step)
   * the plain FP64 form: every cloth stepped on its own, all-FP64, direct
     launches (the denominator of the batched/mixed speedup)
-  * roofline of the dominant kernel (the PCG SpMV, with the direction update
-    and the d.q partial fused in), timed with HIP events on the library's
-    stream: algorithmic bytes per launch / mean launch time vs the 8 TB/s HBM
-    peak
+  * the share of the timed cloth-steps that one launch solved (all of them by
+    default: the matrix stays on the chip for the whole solve)
+  * roofline of the dominant kernel of the solves by launches (the PCG SpMV,
+    with the direction update and the d.q partial fused in), timed by itself
+    with HIP events on the library's stream: algorithmic bytes per launch /
+    mean launch time vs the 8 TB/s HBM peak
   * the CPU baseline: the reference's own CPU step (cBaraffCloth::UpdatePos,
     compiled from its sources -O3 -DNDEBUG into oracle/_ref/ref_cloth), one
     thread, on a bounded sample of the same cloths, each stepped from the
@@ -153,7 +155,7 @@ def time_batch(ms, steps, warmup, graphs=True):
     worst = 0.0
     per_cloth_iters = np.zeros(b.n)
     critical = []
-    fp64_matrix = 0
+    fp64_matrix = one_launch = 0
     t0 = time.perf_counter()
     for _ in range(steps):
         s0 = time.perf_counter()
@@ -164,18 +166,20 @@ def time_batch(ms, steps, warmup, graphs=True):
         critical.append(max(s["pcg_iterations"] + s["outer_iterations"] for s in st))
         per_cloth_iters += [s["pcg_iterations"] for s in st]
         fp64_matrix += sum(s["matrix_fp64"] for s in st)
+        one_launch += sum(s["solve_route"] == 2 for s in st)
         worst = max(worst, max(s["rel_residual"] for s in st))
     total = time.perf_counter() - t0
     b.per_cloth_iters = per_cloth_iters
     b.critical = np.array(critical, dtype=np.float64)
     b.fp64_matrix_fraction = fp64_matrix / float(steps * b.n)
+    b.one_launch_fraction = one_launch / float(steps * b.n)
     b.final_pos = [b.get_pos(i) for i in range(b.n)]
     return b, total, np.array(lat), float(np.mean(iters)), worst
 
 
 def step_bytes(b, fp32=True):
-    """algorithmic bytes of the timed steps' PCG iterations, per iteration of
-    a cloth: its SpMV (matrix block + column index per true block; z, d_prev
+    """algorithmic bytes of the timed steps' PCG iterations as the solves by
+    launches move them, per iteration of a cloth: its SpMV (matrix block + column index per true block; z, d_prev
     read, d, q written per vertex) and update (d, q, r, P read, dx32 read and
     written, r, z written): 40 nnzb + 144 V in the mixed form"""
     total = 0.0
@@ -563,13 +567,16 @@ def main():
         "p99_ms": 1000 * float(np.percentile(lat, 99)),
         "pcg_iterations_mean": iters,
         # the slowest cloth's iterations (and true-residual checks) per step:
-        # a step lasts as long as that cloth's chain of launches
+        # a step lasts at least as long as that cloth's solve
         "critical_iterations_mean": float(np.mean(b.critical)),
         "us_per_critical_iteration": 1e6 * total / float(np.sum(b.critical)),
         # cloth-steps of the timed region whose solve read the FP64 matrix
         # (the mixed form's stall fallback, or its carry-over from an earlier
         # stalled solve of the same cloth)
         "fp64_matrix_fraction": b.fp64_matrix_fraction,
+        # cloth-steps of the timed region that one launch solved; the others
+        # ran the roofline's kernel
+        "one_launch_fraction": b.one_launch_fraction,
         "autotune": {"spmv_lanes_per_row": b.tuning[0], "spmv_staged": b.tuning[1],
                      "spmv_nontemporal": b.tuning[2],
                      "spmv_us": {f: {str(k): float(v) for k, v in t.items()}
@@ -579,6 +586,8 @@ def main():
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "traffic_source": traffic_src,
                      "kernel": kernel_name(*b.tuning[:3], batch_slices(ms)),
+                     "timed": "by itself, as the solves by launches run it (share of the timed "
+                              "cloth-steps: 1 - one_launch_fraction)",
                      "launch_us": us, "alg_bytes": nbytes,
                      # an empty kernel of the same grid and workgroup, launched
                      # back to back: no launch of that shape is shorter, so
@@ -587,10 +596,11 @@ def main():
                      "frac_if_at_floor": nbytes / floor / 1e3 / HBM_PEAK_GBS},
         "whole_step": {"achieved": whole_step_gbs, "unit": "GB/s",
                        "frac": whole_step_gbs / HBM_PEAK_GBS,
-                       "bytes": "per PCG iteration of a cloth 40 nnzb + 144 V (SpMV and update "
-                                "launches), times its iterations over the timed steps, over "
-                                "the timed wall time (assembly and host gaps included in the "
-                                "time, not in the bytes)"},
+                       "bytes": "per PCG iteration of a cloth 40 nnzb + 144 V (what the SpMV and "
+                                "update launches move; a one-launch solve keeps it on the chip, "
+                                "so this is no HBM traffic there), times its iterations over "
+                                "the timed steps, over the timed wall time (assembly and host "
+                                "gaps included in the time, not in the bytes)"},
     }
     b.close()
     x_plain = None
