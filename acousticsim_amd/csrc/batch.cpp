@@ -1411,7 +1411,8 @@ void Batch::solve_cg(const std::function<void()> &again)
             pred_launches_.assign(size(), 0);
         for (int i = 0; i < size(); i++)
         {
-            solved_[i] = resident_.count[i] > 0;
+            // (a cloth that has left it for the FP64 matrix is not)
+            solved_[i] = resident_.count[i] > 0 && host_cg_[2 * i].done;
             if (solved_[i])
                 take_stats(i, host_cg_[2 * i], ROUTE_RESIDENT);
             all &= solved_[i] != 0;

@@ -267,6 +267,7 @@ private:
     void build_resident(const ResidentLists &lists);
     bool solve_resident(const std::function<void()> &again);
     bool all_resident() const;
+    bool w64_size() const;
     bool w64_by_launches() const;
     void free_resident();
     struct ResidentPlan

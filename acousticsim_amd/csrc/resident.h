@@ -77,7 +77,10 @@ struct ResidentLaunch
     int lpr;
     int sets_max, halo_max;     // over the launch's parts (halo_max even)
     int extra;                  // slots of slices past RS_SLOTS that a part keeps in LDS
-    int give_up;                // tests: abort a cloth after this many iterations (0: never)
+    // tests: abort a cloth after this many iterations (0: never); < 0: a cloth
+    // that moves on to the FP64 matrix leaves the launch, for the launches to
+    // finish (one cloth only)
+    int give_up;
     // iterations of a cloth after which its solve pauses until the next launch
     // (0: never); only with one lane per row
     int pause;
@@ -110,7 +113,8 @@ int resident_extra(bool fp32, int sets_max, int halo_max, int wanted);
 // when a launch is given up: after a wait of 2 s in which none of its cloths
 // got on (BW_RESIDENT_WAIT_MS), or at BW_RESIDENT_GIVE_UP iterations of a
 // cloth (tests)
-void resident_limits(ResidentLaunch &a, ResidentCtl &ctl);
+// (w64_leaves: and a cloth leaves it when it moves on to the FP64 matrix)
+void resident_limits(ResidentLaunch &a, ResidentCtl &ctl, bool w64_leaves = false);
 // dynamic LDS bytes of a launch
 size_t resident_lds(bool fp32, int sets_max, int halo_max, int extra);
 // workgroups of the launch that are resident at once on the current device

@@ -784,7 +784,9 @@ k_resident(ResidentLaunch a)
                     room = min(room, uniform(sh_stop - st.total));
                 enough = uniform(fmax(tol2 * st.bb, ip->rel2 * rr));
                 check = false;
-                if (a.give_up > 0 && st.total >= a.give_up)
+                // (as one scalar: 21 x 21 2% faster than as a branch of branches)
+                if (uniform(a.give_up > 0 ? st.total >= a.give_up
+                                          : MIXED && a.give_up < 0 && st.w64 && st.since > 0 && first))
                 {
                     failed = true;
                     break;
@@ -966,8 +968,19 @@ k_resident(ResidentLaunch a)
         }
         if (failed)
         {
-            if (tid == 0)
+            if (tid == 0 && (!MIXED || a.give_up >= 0 || sh_failed))
                 __hip_atomic_store(&a.ctl->aborted, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else if (tid == 0 && pt.slice0 == pt.set0)
+            {
+                // on to the FP64 matrix: the launches form this true residual
+                // again and go on from it
+                CgState st = sh_st;
+                st.start = st.first = 1;
+                st.updates -= 1;
+                store_state(glob(d.cg) + 2 * inst, st);
+                store_state(glob(d.cg) + 2 * inst + 1, st);
+                rb.epoch[inst] = tag;
+            }
             return;
         }
         // the solution and the state for k_update_positions and the host, or

@@ -81,10 +81,10 @@ int resident_extra(bool fp32, int sets_max, int halo_max, int wanted)
     return std::min(wanted, (int)((RS_LDS_MAX - used) / resident_slot_bytes(fp32)));
 }
 
-void resident_limits(ResidentLaunch &a, ResidentCtl &ctl)
+void resident_limits(ResidentLaunch &a, ResidentCtl &ctl, bool w64_leaves)
 {
     ctl.wait_ticks = 100000ULL * (unsigned)std::max(0, env_int("BW_RESIDENT_WAIT_MS", 2000));
-    a.give_up = env_int("BW_RESIDENT_GIVE_UP", 0);
+    a.give_up = env_int("BW_RESIDENT_GIVE_UP", w64_leaves ? -1 : 0);
 }
 
 // Parts of each cloth that fits: its slices in order, as many to a
@@ -269,10 +269,18 @@ bool Batch::all_resident() const
 // 2 of 97 x 97 (296 slices) 12.1 and 11.2, 5 of 65 x 65 (340) 11.6 and 11.2, 2 of
 // 125 x 125 (496) 12.3 and 12.6; 8 of 33 x 33 11.3 and 11.9.  A batch whose other
 // cloths go in the one launch keeps these there, beside them.
+// A cloth alone that moves on to that matrix in mid-solve leaves the launch too
+// (a drape's solve of 51,920 iterations: 604 ms in one launch, 538 by launches
+// from the start, 514 so).
+bool Batch::w64_size() const
+{
+    return kind_ == SolverKind::CG32 && size() < 8 && resident_.most > 1 &&
+           d_.n_slices <= (size() == 1 ? 700 : 350);
+}
+
 bool Batch::w64_by_launches() const
 {
-    if (kind_ != SolverKind::CG32 || size() >= 8 || resident_.most <= 1 ||
-        d_.n_slices > (size() == 1 ? 700 : 350))
+    if (!w64_size())
         return false;
     for (char w : w64_next_)
         if (!w)
@@ -328,7 +336,7 @@ bool Batch::solve_resident(const std::function<void()> &again)
     a.sets_max = rp.sets_max;
     a.halo_max = rp.halo_max;
     a.extra = extra;
-    resident_limits(a, *ctl);
+    resident_limits(a, *ctl, size() == 1 && w64_size());
     int aborted = 0;
     {
         const int grid = std::min(rp.parts, rp.capacity);

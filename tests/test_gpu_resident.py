@@ -124,7 +124,8 @@ def test_fp64_matrix_same_bits(monkeypatch):
                                          ((65, 5), ONE_LAUNCH)])
 def test_fp64_matrix_route(monkeypatch, sides, route):
     """steps that start on the FP64 matrix, by the route that is faster there,
-    and back after the state is set, with the same bits"""
+    and back after the state is set, with the same bits; a cloth alone leaves
+    the launch for that matrix in mid-solve too"""
     cloths = [_grid(n, n, "mixed") for n in sides]
     monkeypatch.setenv("BW_SPMV_LPR", "1")
     # (a 5 x 5 cloth's checks all come within this window)
@@ -141,10 +142,15 @@ def test_fp64_matrix_route(monkeypatch, sides, route):
         for i in range(b.n):
             b.set_state(i, x[i], x[i])
         b.step(1)
-        out.append(([s["solve_route"] for s in st], [b.stats(i)["solve_route"] for i in range(b.n)],
-                    x, [b.get_pos(i) for i in range(b.n)]))
+        st += [b.stats(i) for i in range(b.n)]
+        out.append(([s["solve_route"] for s in st[:b.n]], [s["solve_route"] for s in st[b.n:]],
+                    x, [b.get_pos(i) for i in range(b.n)],
+                    [[s[k] for k in ("pcg_iterations", "outer_iterations", "rel_residual")]
+                     for s in st]))
         b.close()
-    assert out[0][0] == len(sides) * [route] and out[0][1] == len(sides) * [ONE_LAUNCH]
+    again = LAUNCHES if sides == (30,) else ONE_LAUNCH
+    assert out[0][0] == len(sides) * [route] and out[0][1] == len(sides) * [again]
+    assert out[0][4] == out[1][4]
     assert not any(r == ONE_LAUNCH for r in out[1][0] + out[1][1])
     for k in (2, 3):
         for p, q in zip(out[0][k], out[1][k]):
