@@ -352,7 +352,11 @@ __device__ inline ResidentPart uniform_part(const ResidentPart &v)
 // one), so the rest is kept small: what only a true residual needs stays in
 // LDS or memory, what is uniform in scalar registers, and addresses are
 // formed where they are used (here()); with spills to scratch the product
-// alone took 5,500 cycles an iteration instead of 1,150.
+// alone took 5,500 cycles an iteration instead of 1,150.  The compiler keeps
+// 65 to 88 scalars in lanes of a vector register all the same (moved back one
+// by one, most of them in the exchange and at a true residual), and in FP64
+// 154 to 166 of the matrix's registers in the accumulator file, copied back
+// before each product; no variant with 1 or 2 lanes per row spills vectors.
 // REF: the reference's semantics with pcg.hip's rounding (T = double, L = 1):
 // its order of a block's three products, and one set of sums per workgroup.
 template <typename T, int WAVES, int L, bool REF, bool PAUSE = false>
@@ -784,9 +788,14 @@ k_resident(ResidentLaunch a)
                     room = min(room, uniform(sh_stop - st.total));
                 enough = uniform(fmax(tol2 * st.bb, ip->rel2 * rr));
                 check = false;
-                // (as one scalar: 21 x 21 2% faster than as a branch of branches)
-                if (uniform(a.give_up > 0 ? st.total >= a.give_up
-                                          : MIXED && a.give_up < 0 && st.w64 && st.since > 0 && first))
+                bool leave;
+                if constexpr (MIXED) // (one scalar: 21 x 21 4% faster than branches)
+                    leave = uniform(a.give_up > 0
+                                        ? st.total >= a.give_up
+                                        : a.give_up < 0 && st.w64 && st.since > 0 && first);
+                else
+                    leave = a.give_up > 0 && st.total >= a.give_up;
+                if (leave)
                 {
                     failed = true;
                     break;

@@ -8,7 +8,8 @@
 // budget and a state slot, and uploads it (a Batch of one cloth).  A device
 // thread owns the GPU stream: it starts each resident request's next step
 // (element and assembly kernels, solver reset), runs the PCG launches of all
-// solving requests as one multi-batch launch sequence, reads back every
+// solving requests (one launch for those that fit it, which pauses the longer
+// solves; one multi-batch launch sequence for the others), reads back every
 // request's solver state in one copy, finishes the steps whose solve is done
 // (position update), and retires requests that have done all their steps
 // (positions copied to the host, device memory returned to the budget).

@@ -240,10 +240,13 @@ const char *bw_last_error(void);
 
 /* ---- batched stepping (no reference counterpart: many independent cloths
    of uneven size stepped together.  Solves of cloths of up to about 69,000
-   vertices (65,000 in FP64) take one launch for all such cloths of the batch, unless another process keeps the device from running it;
-   the others go by launches per iteration, where from the second step on 8
-   or more cloths solve the ones that needed the most launches in chains of
-   their own on separate streams.  Results are bit-identical either way) -- */
+   vertices (65,000 in FP64) take one launch for all such cloths of the batch,
+   unless another process keeps the device from running it; the others go by
+   launches per iteration, where from the second step on 8 or more such cloths
+   solve the ones that needed the most launches in chains of their own on
+   separate streams.  Fewer than 8 cloths that have stalled and stay on the FP64
+   matrix go by launches too, where those are faster.  Results are bit-identical
+   either way; bw_step_stats::solve_route tells it) ---------------------- */
 
 /* n cloths from n JSON configs; x0s[i] may be NULL */
 int bw_batch_create(const char *const *json_configs, const double *const *x0s,
@@ -325,10 +328,10 @@ int bw_batch_time_launch_floor(bw_batch *b, int reps, double *avg_us);
    bw_batch_step does this by itself when a cloth of the batch solves by
    launches (else it takes 1 lane per row, gathered, cached: the lane count
    sets the rounding that one-launch solves follow, and is kept when the
-   batch falls back to launches).  A variant is 1, 2 or 4 lanes per matrix row; the
-   direction vector gathered from memory per slot, or staged in LDS once
-   per distinct column of a 64-row slice; matrix loads with or without the
-   nontemporal hint.  lanes gets the lanes per row chosen, staged and
+   batch falls back to launches).  A variant is 1, 2 or 4 lanes per matrix
+   row; the direction vector gathered from memory per slot, or staged in LDS
+   once per distinct column of a 64-row slice; matrix loads with or without
+   the nontemporal hint.  lanes gets the lanes per row chosen, staged and
    nontemporal (each may be NULL) 1 if that form was chosen, us (12
    doubles, may be NULL) the mean launch time of variant
    v = (0, 1, 2 for 1, 2, 4 lanes) + 3 * staged + 6 * nontemporal (0 for a
